@@ -115,7 +115,14 @@ ulonglong2 ntt_pair(uint64_t w, uint64_t q) {
         std::memcpy(&b, &wq, 8);
         return ulonglong2{a, b};
     }
-    return shoup_pair(w, q);
+    // w centred (w_c = w or w - q, |w_c| <= q / 2) and s = round(w_c 2^63 / q),
+    // |s| <= 2^62, split as s = hi 2^32 + lo with lo signed
+    const bool neg = w > q / 2;
+    const uint64_t m = neg ? q - w : w;
+    const int64_t t = (int64_t)((((u128)m << 63) + q / 2) / q), s = neg ? -t : t;
+    const int32_t lo = (int32_t)(uint32_t)(uint64_t)s;
+    const uint32_t hi = (uint32_t)((uint64_t)(s - (int64_t)lo) >> 32);
+    return ulonglong2{neg ? (uint64_t)0 - m : m, ((uint64_t)hi << 32) | (uint32_t)lo};
 }
 
 static uint32_t bitrev(uint32_t x, int bits) {
@@ -156,13 +163,16 @@ static void create_coeff_modulus(uint64_t N, const int *bits, size_t count, uint
 // ---------------------------------------------------------------- context
 static uint64_t two32_mod(uint64_t q) { return (uint64_t)(((u128)1 << 32) % q); }
 
-// Second factor pair of a base-conversion entry m for target q: FP64 policy,
-// the pair of m 2^32 mod q (the high half of a wide input); integer policy,
-// m 2^64 mod q (the factor of the Montgomery-accumulated conversion).
+// Second factor pair of a base-conversion entry m for target q: the limbs of
+// m 2^60 mod q as 30-bit halves, and for conversions that do not sum limbs, FP64
+// policy: m 2^32 mod q as a double (the high half of a wide input); integer
+// policy: m 2^64 mod q (128-bit sums).
 static ulonglong2 bconv_pair1(uint64_t m, uint64_t q) {
-    if (q < kF64PrimeBound) return ntt_pair(mulmod(m, two32_mod(q), q), q);
+    const uint64_t mm = mulmod(m, (uint64_t)(((u128)1 << 60) % q), q);
+    const uint64_t limbs = ((mm >> 30) << 32) | (mm & ((1ull << 30) - 1));
+    if (q < kF64PrimeBound) return ulonglong2{limbs, ntt_pair(mulmod(m, two32_mod(q), q), q).x};
     const uint64_t r64 = (uint64_t)((((u128)1 << 64) - 1) % q + 1) % q;  // 2^64 mod q
-    return ulonglong2{mulmod(m, r64, q), 0};
+    return ulonglong2{limbs, mulmod(m, r64, q)};
 }
 
 static uint64_t prod_mod(const uint64_t *m, size_t n, size_t skip, uint64_t p) {

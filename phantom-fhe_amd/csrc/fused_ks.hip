@@ -35,8 +35,9 @@
 // split t = h 2^32 + l and converted as h [m 2^32]_q + l m.  Each product is
 // within (-0.875 q, 0.875 q) (|t w / q| < 2^50, so fl(t wq) is within 3/8 of
 // the true quotient); the sum is reduced whenever the next product could take
-// it past 7 x 0.875 q, which keeps every partial sum below 2^53.  Targets q >= 2^50 use integer
-// Shoup products, each in [0, 2q), summed with a conditional subtraction.
+// it past 7 x 0.875 q, which keeps every partial sum below 2^53.  Targets
+// q >= 2^50, and FP64 targets with a wide input, sum 30-bit limb products
+// (bconv_limbs).
 #include <algorithm>
 
 #include "internal.h"
@@ -88,11 +89,12 @@ struct BconvCols {
     // every factor is 1 (ModUp with alpha = 1: Q_b = q_i; the rescale's single
     // input): a lone input below 2^50 is then only reduced, not multiplied
     uint32_t unit = 0;
-    // integer-policy targets with two inputs or more: 128-bit sums of the
-    // inputs times the factors in Montgomery form (pair 1, m 2^64 mod q) and
-    // one Montgomery reduction (the context's constants -q^-1 mod 2^64); set by
-    // the launcher when every input sum stays below 2^64, else null (Shoup)
+    // the context's Montgomery constants (x = -q^-1 mod 2^64)
     const ulonglong2 *mont = nullptr;
+    uint32_t sum128 = 0;  // kWide: the integer targets' sums of inputs stay below 2^64
+    // the inputs of primes of 50 bits or more are stored as 30-bit halves
+    // (hi 2^32 + lo), NttLaunch::split30
+    uint32_t split30 = 0;
     // position -> item table (a permutation of the launch's positions) built
     // for sched_grid workgroups over sched_total positions; the launcher drops
     // it when its launch differs.  null: position p runs item p
@@ -111,27 +113,160 @@ __device__ __forceinline__ const ulonglong2 *bc_of(const BconvCols &a, uint32_t 
     return a.bc + (size_t)g * a.bc_gstride + ((size_t)i * a.bc_istride + j) * 2;
 }
 
-template <class A, int S1, int S2>
+// A residue at a wave-uniform base and a 32-bit byte offset (scalar base plus
+// vector offset addressing).
+__device__ __forceinline__ uint64_t ld_at(const uint64_t *base, uint32_t off) {
+    return *reinterpret_cast<const uint64_t *>(reinterpret_cast<const char *>(base) + (size_t)off);
+}
+
+constexpr uint32_t kLimbInputs = 7;
+
+// sum_i t_i m_i mod q, in [0, (n_in + 1) q), for elements F + T e of the
+// thread's column, by 30-bit limbs: t = t1 2^30 + t0 and the factor in
+// Montgomery form, m 2^60 mod q = m1 2^30 + m0, so a product is four 32-bit
+// multiply-adds into three 64-bit sums, with no carries to move (a 128-bit sum
+// takes about 13 instructions a product); two 30-bit Montgomery steps then
+// divide by 2^60.  With t, q < 2^60 and n <= 7: the middle sum stays below
+// (2 n + 1) 2^60 + 2^35 < 2^64 and the result below n q^2 / 2^60 + q.
+// Inputs of wide primes come split from the INTT; narrower ones are split here.
+// Measured at N = 2^16 with the columns pass it feeds: 14 polys of 6 wide inputs to
+// 28 wide targets plus 5 digits of 6 to 34, 322 us with 128-bit sums, 270 us.
+template <int S1, int S2>
+__device__ __forceinline__ void bconv_limbs(const BconvCols &a, const NttTables &t, uint64_t q, uint32_t g, uint32_t j,
+                                            uint32_t prow, uint32_t n_in, uint32_t row0, const uint64_t *in,
+                                            uint32_t off, uint64_t (&x)[Sub<S1>::E]) {
+    using G = Geo<S1, S2>;
+    using SB = Sub<S1>;
+    constexpr uint32_t M30 = (1u << 30) - 1;
+    constexpr int H = SB::E < 4 ? SB::E : 4;  // elements at a time: 3 H 64-bit sums
+    const uint32_t qn = (uint32_t)ld_const(reinterpret_cast<const uint64_t *>(a.mont + prow)) & M30;
+    const uint32_t q0 = (uint32_t)q & M30, q1 = (uint32_t)(q >> 30);
+    // the next input's residues (or the next group's first) are requested
+    // before this input's products
+    uint64_t v[H];
+#pragma unroll
+    for (int e = 0; e < H; e++) v[e] = ld_at(in + (size_t)SB::T * e * G::N2, off);
+#pragma unroll
+    for (int h = 0; h < SB::E; h += H) {
+        __builtin_amdgcn_sched_barrier(0);
+        uint64_t s0[H], s1[H], s2[H];
+#pragma unroll
+        for (int e = 0; e < H; e++) s0[e] = s1[e] = s2[e] = 0;
+#pragma nounroll
+        for (uint32_t i = 0; i < n_in; i++) {
+            const uint64_t m = ld_const(reinterpret_cast<const uint64_t *>(bc_of(a, g, i, j) + 1));
+            const uint32_t m0 = (uint32_t)m, m1 = (uint32_t)(m >> 32);
+            const bool split = a.split30 && ld_const(t.mod + bconv_in_row(a, row0, i)) >= kF64PrimeBound;
+            const bool more = i + 1 < n_in;
+            const uint64_t *next = in + (more ? (size_t)(i + 1) * G::N + (size_t)SB::T * h * G::N2
+                                              : (size_t)SB::T * (h + H < SB::E ? h + H : h) * G::N2);
+            uint64_t nv[H];
+#pragma unroll
+            for (int e = 0; e < H; e++) nv[e] = ld_at(next + (size_t)SB::T * e * G::N2, off);
+            if (!split) {
+#pragma unroll
+                for (int e = 0; e < H; e++) v[e] = ((v[e] >> 30) << 32) | ((uint32_t)v[e] & M30);
+            }
+#pragma unroll
+            for (int e = 0; e < H; e++) {
+                const uint32_t t0 = (uint32_t)v[e], t1 = (uint32_t)(v[e] >> 32);
+                s0[e] += (uint64_t)t0 * m0;
+                s1[e] += (uint64_t)t0 * m1;
+                s1[e] += (uint64_t)t1 * m0;
+                s2[e] += (uint64_t)t1 * m1;
+                v[e] = nv[e];
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < H; e++) {
+            const uint32_t k0 = ((uint32_t)s0[e] * qn) & M30;
+            s0[e] += (uint64_t)k0 * q0;
+            s1[e] += (uint64_t)k0 * q1 + (s0[e] >> 30);
+            const uint32_t k1 = ((uint32_t)s1[e] * qn) & M30;
+            s1[e] += (uint64_t)k1 * q0;
+            x[h + e] = s2[e] + (uint64_t)k1 * q1 + (s1[e] >> 30);
+            asm volatile("" : "+v"(x[h + e]));  // formed here: not both groups' sums at once
+        }
+    }
+}
+
+// What a launch's conversions can be, chosen by the launcher: kOne a single
+// input each; kLimbs sums that may take 30-bit limbs (every prime below 2^60, at
+// most kLimbInputs inputs); kWide the rest (128-bit sums for the integer targets
+// when every input sum stays below 2^64).  One kernel each: in one kernel the
+// branches' values together did not fit the registers, and the few spilled
+// ones, reloaded once an item, waited behind the stores of the item before
+// (L = 35 conversions 242 -> 285 us).
+enum BconvKind { kOne, kLimbs, kWide };
+
+template <class A, int S1, int S2, int KIND>
 __device__ __forceinline__ void bconv_source(const BconvCols &a, const NttTables &t, const A &ar, uint32_t mi,
-                                             uint32_t g, uint32_t j, uint32_t tile, uint32_t prow,
+                                             uint32_t g, uint32_t j, uint32_t tile, uint32_t prow, uint32_t tid,
                                              typename A::T (&x)[Sub<S1>::E]) {
     using G = Geo<S1, S2>;
     using SB = Sub<S1>;
-    const uint32_t c = threadIdx.x % kCols, F = threadIdx.x / kCols;
-    const uint32_t n_in = g + 1 == a.groups ? a.n_in_last : a.n_in;
-    const uint64_t *base = a.in + (size_t)mi * a.in_bstride + (size_t)g * a.in_gstride + tile * kCols + c;
-    const uint32_t row0 = a.in_row0 + g * a.in_row_step;
-    if constexpr (A::kF64) {
-        if (a.unit && n_in == 1 && t.mod[bconv_in_row(a, row0, 0)] < kF64PrimeBound) {
-            // x = v mod q with v < 2^50: the FMA remainder of the nearest
-            // quotient is exact and within (0.5 + 2^-20) q of zero
+    const uint32_t c = tid % kCols, F = tid / kCols;
+    const uint32_t n_in = KIND == kOne ? 1 : g + 1 == a.groups ? a.n_in_last : a.n_in;
+    const uint64_t *in = a.in + (size_t)mi * a.in_bstride + (size_t)g * a.in_gstride + tile * kCols;
+    const uint32_t off = (F * G::N2 + c) * 8;
+    // one input's residues, all requested before the first is used
+    uint64_t v[SB::E];
+    const auto request = [&](uint32_t i) {
 #pragma unroll
-            for (int e = 0; e < SB::E; e++) {
-                x[e] = ar.load(base[(size_t)(F + SB::T * e) * G::N2]);
-                ar.reduce(x[e]);
+        for (int e = 0; e < SB::E; e++) v[e] = ld_at(in + (size_t)i * G::N + (size_t)SB::T * e * G::N2, off);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    const uint32_t row0 = a.in_row0 + g * a.in_row_step;
+    const auto mod_of = [&](uint32_t i) { return ld_const(t.mod + bconv_in_row(a, row0, i)); };
+    if constexpr (KIND == kOne) {
+        request(0);
+        const uint64_t m = mod_of(0);
+        if constexpr (A::kF64) {
+            if (a.unit && m < kF64PrimeBound) {
+                // x = v mod q with v < 2^50: the FMA remainder of the nearest
+                // quotient is exact and within (0.5 + 2^-20) q of zero
+#pragma unroll
+                for (int e = 0; e < SB::E; e++) x[e] = ar.load(v[e]);
+            } else {
+                const ulonglong2 *f = bc_of(a, g, 0, j);
+                const double w0 = ArithF64::as_f(f[0].x), wq0 = ArithF64::as_f(f[0].y);
+                const double w1 = ArithF64::as_f(f[1].y), wq1 = w1 * ar.qinv;
+#pragma unroll
+                for (int e = 0; e < SB::E; e++)
+                    x[e] = ar.mulw((double)(uint32_t)(v[e] >> 32), w1, wq1) + ar.mulw((double)(uint32_t)v[e], w0, wq0);
             }
+        } else {
+            const bool small = a.unit && !ar.tight && m <= 8 * ar.q;  // v mod q with v < 8 q
+            const ulonglong2 f = ld_const(bc_of(a, g, 0, j));
+#pragma unroll
+            for (int e = 0; e < SB::E; e++) x[e] = small ? v[e] : ar.mulw(v[e], f);
+        }
+#pragma unroll
+        for (int e = 0; e < SB::E; e++) ar.reduce(x[e]);
+        return;
+    }
+    if constexpr (KIND == kLimbs) {
+        // an input of a wide prime takes two FP64 products (16 instructions),
+        // a narrow one 9; by limbs either takes 4 to 6, and the two Montgomery
+        // steps 14 an element: limbs as soon as one input is wide
+        bool limbs = !A::kF64;
+        if constexpr (A::kF64)
+            for (uint32_t i = 0; i < n_in; i++) limbs = limbs || mod_of(i) >= kF64PrimeBound;
+        if (limbs) {
+            if constexpr (A::kF64) {
+                bconv_limbs<S1, S2>(a, t, (uint64_t)ar.q, g, j, prow, n_in, row0, in, off, v);
+#pragma unroll
+                for (int e = 0; e < SB::E; e++)  // below 8 q < 2^53: exact
+                    x[e] = __fma_rn((double)(uint32_t)(v[e] >> 32), 4294967296.0, (double)(uint32_t)v[e]);
+            } else {
+                bconv_limbs<S1, S2>(a, t, ar.q, g, j, prow, n_in, row0, in, off, x);
+            }
+#pragma unroll
+            for (int e = 0; e < SB::E; e++) ar.reduce(x[e]);
             return;
         }
+    }
+    if constexpr (A::kF64) {
         double acc[SB::E];
 #pragma unroll
         for (int e = 0; e < SB::E; e++) acc[e] = 0.0;
@@ -140,8 +275,8 @@ __device__ __forceinline__ void bconv_source(const BconvCols &a, const NttTables
             const ulonglong2 *f = bc_of(a, g, i, j);
             const ulonglong2 f0 = f[0];
             const double w0 = ArithF64::as_f(f0.x), wq0 = ArithF64::as_f(f0.y);
-            const uint64_t *src = base + (size_t)i * G::N;
-            const bool wide = t.mod[bconv_in_row(a, row0, i)] >= kF64PrimeBound;
+            const bool wide = KIND == kWide && mod_of(i) >= kF64PrimeBound;
+            request(i);
             if (units + (wide ? 2u : 1u) > 7u) {
 #pragma unroll
                 for (int e = 0; e < SB::E; e++) ar.reduce(acc[e]);
@@ -149,16 +284,14 @@ __device__ __forceinline__ void bconv_source(const BconvCols &a, const NttTables
             }
             units += wide ? 2u : 1u;
             if (wide) {
-                const ulonglong2 f1 = f[1];
-                const double w1 = ArithF64::as_f(f1.x), wq1 = ArithF64::as_f(f1.y);
+                const double w1 = ArithF64::as_f(f[1].y), wq1 = w1 * ar.qinv;
 #pragma unroll
-                for (int e = 0; e < SB::E; e++) {
-                    const uint64_t v = src[(size_t)(F + SB::T * e) * G::N2];
-                    acc[e] += ar.mulw((double)(uint32_t)(v >> 32), w1, wq1) + ar.mulw((double)(uint32_t)v, w0, wq0);
-                }
+                for (int e = 0; e < SB::E; e++)
+                    acc[e] += ar.mulw((double)(uint32_t)(v[e] >> 32), w1, wq1) +
+                              ar.mulw((double)(uint32_t)v[e], w0, wq0);
             } else {
 #pragma unroll
-                for (int e = 0; e < SB::E; e++) acc[e] += ar.mulw(ar.load(src[(size_t)(F + SB::T * e) * G::N2]), w0, wq0);
+                for (int e = 0; e < SB::E; e++) acc[e] += ar.mulw(ar.load(v[e]), w0, wq0);
             }
         }
 #pragma unroll
@@ -166,44 +299,43 @@ __device__ __forceinline__ void bconv_source(const BconvCols &a, const NttTables
             ar.reduce(acc[e]);
             x[e] = acc[e];
         }
-    } else {
-        const uint64_t q = ar.q, q2 = ar.q2;
-        if (a.mont && n_in >= 2) {
+    } else if constexpr (KIND == kWide) {
+        const uint64_t q = ar.q;
+        if (a.sum128) {
             // sum_i t_i (m_i 2^64 mod q) < q sum_i t_i < q 2^64, so one
-            // Montgomery reduction gives sum_i t_i m_i mod q in [0, 2q): 4
-            // multiplies per input and 7 for the reduction, against a
-            // 10-multiply Shoup product per input
+            // Montgomery reduction gives sum_i t_i m_i mod q in [0, 2q), taken
+            // to [-q, q)
             const uint64_t qn = ld_const(reinterpret_cast<const uint64_t *>(a.mont + prow));
             U128 acc[SB::E];
 #pragma unroll
             for (int e = 0; e < SB::E; e++) acc[e] = U128{0, 0};
             for (uint32_t i = 0; i < n_in; i++) {
-                const uint64_t mm = ld_const(reinterpret_cast<const uint64_t *>(bc_of(a, g, i, j) + 1));
-                const uint64_t *src = base + (size_t)i * G::N;
+                const uint64_t mm = ld_const(reinterpret_cast<const uint64_t *>(bc_of(a, g, i, j) + 1) + 1);
 #pragma unroll
-                for (int e = 0; e < SB::E; e++) mac(acc[e], src[(size_t)(F + SB::T * e) * G::N2], mm);
+                for (int e = 0; e < SB::E; e++)
+                    mac(acc[e], ld_at(in + (size_t)i * G::N + (size_t)SB::T * e * G::N2, off), mm);
             }
 #pragma unroll
-            for (int e = 0; e < SB::E; e++) x[e] = mont_reduce(acc[e], q, qn);
+            for (int e = 0; e < SB::E; e++) x[e] = mont_reduce(acc[e], q, qn) - q;
             return;
         }
-        uint64_t acc[SB::E];
 #pragma unroll
-        for (int e = 0; e < SB::E; e++) acc[e] = 0;
+        for (int e = 0; e < SB::E; e++) x[e] = 0;
         for (uint32_t i = 0; i < n_in; i++) {
-            const ulonglong2 f0 = bc_of(a, g, i, j)[0];
-            const uint64_t *src = base + (size_t)i * G::N;
+            const ulonglong2 f0 = ld_const(bc_of(a, g, i, j));
+            request(i);
 #pragma unroll
-            for (int e = 0; e < SB::E; e++)
-                acc[e] = csub(acc[e] + shoup_lazy(src[(size_t)(F + SB::T * e) * G::N2], f0.x, f0.y, q), q2);
+            for (int e = 0; e < SB::E; e++) {
+                x[e] += ar.mulw(v[e], f0);  // 0.5 q + 1.6 q
+                ar.reduce(x[e]);
+            }
         }
-#pragma unroll
-        for (int e = 0; e < SB::E; e++) x[e] = acc[e];
     }
 }
 
-template <int S1, int S2>
-__global__ void __launch_bounds__((Geo<S1, S2>::COL_THREADS)) k_bconv_cols(BconvCols a, NttTables t) {
+template <int S1, int S2, int KIND>
+__global__ void __launch_bounds__((Geo<S1, S2>::COL_THREADS)) __attribute__((amdgpu_waves_per_eu(S1 >= 7 ? 4 : 3, S1 >= 7 ? 4 : 3)))
+k_bconv_cols(BconvCols a, NttTables t) {
     using G = Geo<S1, S2>;
     using SB = Sub<S1>;
     __shared__ double lds[G::COL_LDS];
@@ -214,6 +346,9 @@ __global__ void __launch_bounds__((Geo<S1, S2>::COL_THREADS)) k_bconv_cols(Bconv
         const uint32_t w = a.sched ? ld_const(a.sched + p) : p;
         uint32_t gt, j;
         if (!grouped_item(w, NG, a.J, gt, j)) continue;
+        // opaque: what is formed from it is not kept from item to item
+        uint32_t tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
         const uint32_t mg = gt / G::COL_TILES, tile = gt % G::COL_TILES;
         const uint32_t mi = mg / a.groups, g = mg % a.groups;
         if (a.skip && j >= g * a.n_in && j < g * a.n_in + (g + 1 == a.groups ? a.n_in_last : a.n_in)) continue;
@@ -226,19 +361,19 @@ __global__ void __launch_bounds__((Geo<S1, S2>::COL_THREADS)) k_bconv_cols(Bconv
         if (q < kF64PrimeBound) {
             const ArithF64 ar(q);
             double x[SB::E];
-            bconv_source<ArithF64, S1, S2>(a, t, ar, mi, g, j, tile, prow, x);
+            bconv_source<ArithF64, S1, S2, KIND>(a, t, ar, mi, g, j, tile, prow, tid, x);
             st.store(twl);
             __syncthreads();
-            fwd_cols_core<ArithF64, S1, S2>(x, ar, twl, lds);
-            fwd_cols_store<ArithF64, S1, S2>(x, ar, tile, olimb);
+            fwd_cols_core<ArithF64, S1, S2>(x, ar, twl, lds, tid);
+            fwd_cols_store<ArithF64, S1, S2>(x, ar, tile, olimb, tid);
         } else {
             const ArithInt ar(q);
             uint64_t x[SB::E];
-            bconv_source<ArithInt, S1, S2>(a, t, ar, mi, g, j, tile, prow, x);
+            bconv_source<ArithInt, S1, S2, KIND>(a, t, ar, mi, g, j, tile, prow, tid, x);
             st.store(twl);
             __syncthreads();
-            fwd_cols_core<ArithInt, S1, S2>(x, ar, twl, reinterpret_cast<uint64_t *>(lds));
-            fwd_cols_store<ArithInt, S1, S2>(x, ar, tile, olimb);
+            fwd_cols_core<ArithInt, S1, S2>(x, ar, twl, reinterpret_cast<uint64_t *>(lds), tid);
+            fwd_cols_store<ArithInt, S1, S2>(x, ar, tile, olimb, tid);
         }
         __syncthreads();
     }
@@ -355,7 +490,10 @@ struct WsGeo {
     // N2 = 256, where the table (16 KiB) still leaves 3 workgroups per CU
     static constexpr bool USE_TAB = S2 <= 8;
     static constexpr int TAB_ROW = G::N2 - 1;
-    static constexpr int TAB = USE_TAB ? ROWS * TAB_ROW : 0;
+    // integer policy: the same place holds the rows' twiddle pairs of every
+    // stage but the last (TWI slots a row, 2^(S2-1) - 1 used)
+    static constexpr int TWI = 1 << (S2 - 1);
+    static constexpr int TAB = USE_TAB ? (TAB_ROW > 2 * TWI ? TAB_ROW : 2 * TWI) * ROWS : 0;
     static_assert(!USE_TAB || 2 * TW <= ROWS * G::ROW_PITCH, "staged entries must fit in one tile buffer");
     // accumulate role: outputs per thread, threads per output, elements per thread and output
     static constexpr int NO = HALF >= 128 ? 1 : 2;
@@ -374,17 +512,59 @@ __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Integer twiddles of one row: entry i of stage g at 2^g - 1 + i in LDS for
+// every stage but the last, whose entries a thread holds (element block F:
+// N of them).
+template <int S>
+struct WsTw {
+    const ulonglong2 *w;
+    uint32_t F;
+    __device__ __forceinline__ ulonglong2 at(int g, int i) const { return w[(1 << g) - 1 + i]; }
+};
+template <int S>
+struct WsTwLast {
+    static constexpr int N = Sub<S>::E / 2;
+    ulonglong2 w[N];
+};
+template <int S>
+struct WsTwB {
+    const WsTw<S> &t;
+    const WsTwLast<S> &l;
+    __device__ __forceinline__ ulonglong2 at(int g, int i) const {
+        return g == S - 1 ? l.w[i] : t.w[(1 << g) - 1 + (t.F << (Sub<S>::LE - S + g)) + i];
+    }
+};
+
 template <class A, int S1, int S2>
 __device__ __forceinline__ void ws_transform(const InnerRows &a, const NttTables &t, const A &ar, uint32_t r,
                                              uint32_t prow, uint32_t k1, uint32_t rr, const ulonglong2 *tws,
-                                             const double *tab, typename A::T *b0, typename A::T *b1, uint32_t db,
-                                             uint32_t de) {
+                                             const double *tab, ulonglong2 *ra, typename A::T *b0, typename A::T *b1, uint32_t db,
+                                             uint32_t de, uint32_t tid) {
     using G = Geo<S1, S2>;
     using W = WsGeo<S1, S2>;
     using SB = Sub<S2>;
     using T = typename A::T;
-    const uint32_t F = (threadIdx.x % W::HALF) % SB::T;
+    const uint32_t F = (tid % W::HALF) % SB::T;
     const size_t rowoff = (size_t)k1 * G::N2 + F;
+    // integer policy: the row's twiddles once per item, before any prefetch
+    // (loads complete in issue order: read inside the rounds they waited for
+    // the next digit's tile, a whole memory latency a digit): all stages but
+    // the last in LDS (written and read within the row's wave), the last one's
+    // in registers
+    constexpr bool PRE = !A::kF64 && W::USE_TAB;
+    const WsTw<S2> wt{ra + rr * W::TWI, F};
+    WsTwLast<S2> wl;
+    if constexpr (PRE) {
+        const ulonglong2 *tw = t.tw + (size_t)prow * G::N;
+        for (uint32_t i = F; i < (uint32_t)W::TWI - 1; i += SB::T) {
+            const uint32_t g = 31 - __builtin_clz(i + 1);
+            ra[rr * W::TWI + i] = tw_at(tw, ((G::N1 + k1) << g) + (i + 1 - (1u << g)));
+        }
+#pragma unroll
+        for (int i = 0; i < WsTwLast<S2>::N; i++)
+            wl.w[i] = tw_at(tw, ((G::N1 + k1) << (S2 - 1)) + F * WsTwLast<S2>::N + i);
+        wave_lds_sync();
+    }
     uint64_t nraw[SB::E];
     bool nown;
     {
@@ -414,6 +594,8 @@ __device__ __forceinline__ void ws_transform(const InnerRows &a, const NttTables
                 uint32_t kr = rr;
                 asm volatile("" : "+v"(kr));
                 fwd_round_a_derived<S2, W::ROWS>(x, ar, tws, tws + W::TW_RB, kr);
+            } else if constexpr (PRE) {
+                fwd_round_a_int<S2>(x, ar, wt);
             } else {
                 uint32_t kr = k1, pr = prow;
                 asm volatile("" : "+v"(kr), "+s"(pr));
@@ -434,6 +616,8 @@ __device__ __forceinline__ void ws_transform(const InnerRows &a, const NttTables
                 uint32_t kr = rr;
                 asm volatile("" : "+v"(kr));
                 fwd_round_b_derived<S2, W::ROWS>(x, ar, tws, tws + W::TW_RB, kr, F);
+            } else if constexpr (PRE) {
+                fwd_round_b_int<S2>(x, ar, WsTwB<S2>{wt, wl});
             } else {
                 uint32_t kr = k1, pr = prow;
                 asm volatile("" : "+v"(kr), "+s"(pr));
@@ -441,7 +625,12 @@ __device__ __forceinline__ void ws_transform(const InnerRows &a, const NttTables
             }
             wave_lds_sync();
 #pragma unroll
-            for (int e = 0; e < SB::E; e++) buf[rpad(F * SB::E + e)] = x[e];
+            for (int e = 0; e < SB::E; e++) {
+                if constexpr (A::kF64)
+                    buf[rpad(F * SB::E + e)] = x[e];
+                else
+                    buf[rpad(F * SB::E + e)] = ar.unsign(x[e]);
+            }
         } else {
 #pragma unroll
             for (int e = 0; e < SB::E; e++) buf[rpad(F + SB::T * e)] = x[e];
@@ -453,8 +642,9 @@ __device__ __forceinline__ void ws_transform(const InnerRows &a, const NttTables
 
 // Product of digit d's transformed element x (lazy) with key limb value w,
 // accumulated into acc: FP64 policy exact products (acc reduced every second
-// digit); integer policy Montgomery products x w 2^-64, each in [0, 2q), summed
-// in [0, 2q) (ws_sum turns the sum back into sum x w mod q).
+// digit); integer policy Montgomery products x w 2^-64 (x made nonnegative by
+// the transform), each in [0, 2q), summed in [0, 2q) (ws_sum turns the sum
+// back into sum x w mod q).
 template <class A>
 __device__ __forceinline__ void ws_mac(const A &ar, typename A::T &acc, typename A::T x, uint64_t w, ulonglong2 mt) {
     if constexpr (A::kF64) {
@@ -462,7 +652,7 @@ __device__ __forceinline__ void ws_mac(const A &ar, typename A::T &acc, typename
         const double wd = ar.load(w);
         acc += ar.mulw(x, wd, wd * ar.qinv);
     } else {
-        acc = csub(acc + mont_mul(x, w, ar.q, mt.x), ar.q2);
+        acc = csub(acc + mont_mul(x, w, ar.q, mt.x), 2 * ar.q);
     }
 }
 
@@ -472,7 +662,7 @@ __device__ __forceinline__ uint64_t ws_sum(const A &ar, typename A::T acc, ulong
     if constexpr (A::kF64)
         return ar.store(acc);
     else
-        return ar.store(mont_mul(acc, mt.y, ar.q, mt.x));  // (sum 2^-64) 2^128 2^-64
+        return csub(mont_mul(acc, mt.y, ar.q, mt.x), ar.q);  // (sum 2^-64) 2^128 2^-64
 }
 
 // Output k of limb r at offset off (within the limb): the canonical sum v, or
@@ -496,12 +686,12 @@ __device__ __forceinline__ void ws_out(const InnerRows &a, uint32_t k, uint32_t 
 template <class A, int S1, int S2>
 __device__ __forceinline__ void ws_accumulate(const InnerRows &a, const A &ar, uint32_t r, uint32_t prow,
                                               uint32_t tile, const typename A::T *B0, const typename A::T *B1,
-                                              uint32_t db, uint32_t de, uint64_t *part) {
+                                              uint32_t db, uint32_t de, uint64_t *part, uint32_t tid) {
     using G = Geo<S1, S2>;
     using W = WsGeo<S1, S2>;
     using T = typename A::T;
     constexpr int NO = W::NO, AE = W::AE, TPO = W::TPO;
-    const uint32_t u = threadIdx.x - W::HALF;
+    const uint32_t u = tid - W::HALF;
     const uint32_t lane = u % TPO, kf = NO == 1 ? u / TPO : 0;  // kf: this thread's output when NO == 1
     const size_t tbase = (size_t)tile * W::ROWS * G::N2 + lane;  // element offset within a limb
     const size_t keyrow = (size_t)prow * G::N + tbase;
@@ -588,9 +778,19 @@ __device__ __forceinline__ void ws_item(const InnerRows &a0, const NttTables &t,
                                         uint32_t de, uint64_t *part, double *lds, ulonglong2 *tws) {
     using G = Geo<S1, S2>;
     using W = WsGeo<S1, S2>;
+    // Opaque, so that nothing derived from the thread index is computed once
+    // for all items and kept: those values filled the registers of both
+    // policies' digit loops and were spilled (22 instead of 58 with the integer
+    // twiddles held; with them and one copy of this code, N = 2^16: 24 + 4
+    // targets of 6 digits 95.8 -> 93.1 us, 20 + 4 of 5 58.5 -> 50.6 us, 36
+    // of 35 431 -> 421 us).
+    uint32_t tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
     double *tab = lds + W::LDS;
-    const bool transform = threadIdx.x < W::HALF;
-    const uint32_t rr = (threadIdx.x % W::HALF) / Sub<S2>::T;
+    // the integer policy's staged twiddles take the table's place
+    ulonglong2 *ra = reinterpret_cast<ulonglong2 *>(tab);
+    const bool transform = tid < W::HALF;
+    const uint32_t rr = (tid % W::HALF) / Sub<S2>::T;
     uint32_t mi, w;
     ws_decode(a0, w0, W::TILES, mi, w);
     InnerRows a = a0;
@@ -617,7 +817,7 @@ __device__ __forceinline__ void ws_item(const InnerRows &a0, const NttTables &t,
             // this item's rows' base factors rb[g][tile ROWS + i] and the small table
             const ulonglong2 *rb = t.rb_fw + (size_t)prow * S2 * G::N1 + tile * W::ROWS;
             const ulonglong2 *small = t.small_fw + (size_t)prow * kSmall;
-            for (uint32_t i = threadIdx.x; i < (uint32_t)W::TW; i += W::HALF)
+            for (uint32_t i = tid; i < (uint32_t)W::TW; i += W::HALF)
                 tws[i] = i < (uint32_t)W::TW_RB ? rb[(i / W::ROWS) * G::N1 + i % W::ROWS] : small[i - W::TW_RB];
         }
         __syncthreads();
@@ -625,21 +825,22 @@ __device__ __forceinline__ void ws_item(const InnerRows &a0, const NttTables &t,
         // digit): each digit's rows pass then reads them instead of deriving
         // them, which shortens the transform role, the longer of the two
         if constexpr (W::USE_TAB) {
-            build_row_tab<S2, W::ROWS>(tab, ArithF64(q), tws, tws + W::TW_RB, threadIdx.x, W::THREADS);
+            build_row_tab<S2, W::ROWS>(tab, ArithF64(q), tws, tws + W::TW_RB, tid, W::THREADS);
             __syncthreads();
         }
         if (transform)
-            ws_transform<ArithF64, S1, S2>(a, t, ArithF64(q), r, prow, k1, rr, tws, tab, b0, b1, db, de);
+            ws_transform<ArithF64, S1, S2>(a, t, ArithF64(q), r, prow, k1, rr, tws, tab, ra, b0, b1, db, de, tid);
         else
             ws_accumulate<ArithF64, S1, S2>(a, ArithF64(q), r, prow, tile, lds, lds + W::ROWS * G::ROW_PITCH, db, de,
-                                             part);
+                                             part, tid);
     } else {
         uint64_t *b0 = reinterpret_cast<uint64_t *>(lds) + rr * G::ROW_PITCH, *b1 = b0 + W::ROWS * G::ROW_PITCH;
         if (transform)
-            ws_transform<ArithInt, S1, S2>(a, t, ArithInt(q), r, prow, k1, rr, tws, tab, b0, b1, db, de);
+            ws_transform<ArithInt, S1, S2>(a, t, ArithInt(q), r, prow, k1, rr, tws, tab, ra, b0, b1, db, de, tid);
         else
             ws_accumulate<ArithInt, S1, S2>(a, ArithInt(q), r, prow, tile, reinterpret_cast<uint64_t *>(lds),
-                                             reinterpret_cast<uint64_t *>(lds) + W::ROWS * G::ROW_PITCH, db, de, part);
+                                             reinterpret_cast<uint64_t *>(lds) + W::ROWS * G::ROW_PITCH, db, de, part,
+                                             tid);
     }
 }
 
@@ -733,20 +934,22 @@ k_inner_ws(InnerRows a0, NttTables t) {
     ulonglong2 *tws = reinterpret_cast<ulonglong2 *>(lds + (W::USE_TAB ? W::ROWS * Geo<S1, S2>::ROW_PITCH : W::LDS));
     const uint32_t total = a0.batch * a0.QlP * W::TILES;
     const uint32_t full = a0.full < total ? a0.full : total;
-    for (uint32_t i = blockIdx.x; i < full; i += gridDim.x) {
-        const uint32_t w0 = full - 1 - i;  // the last items (the longest) first
-        ws_item<S1, S2>(a0, t, w0, 0, a0.beta, nullptr, lds, tws);
-        __syncthreads();
-    }
-    if (a0.rem == 0) return;
+    constexpr size_t PS = (size_t)2 * W::ROWS * Geo<S1, S2>::N2;
     const uint32_t g = gridDim.x - 1 - blockIdx.x;
     const uint32_t u = g / kXcds, c = u % a0.kch;
     const uint32_t j = (u / a0.kch) * kXcds + g % kXcds;
-    if (j >= a0.rem) return;
-    constexpr size_t PS = (size_t)2 * W::ROWS * Geo<S1, S2>::N2;
     const uint64_t *parts = a0.partial + (size_t)j * a0.kch * PS;
-    ws_item<S1, S2>(a0, t, full + j, c * a0.beta / a0.kch, (c + 1) * a0.beta / a0.kch,
-                    a0.partial + ((size_t)j * a0.kch + c) * PS, lds, tws);
+    // one call for whole items and the chunk: two copies of the item's code
+    // did not fit the instruction cache together
+    for (uint32_t i = blockIdx.x;; i += gridDim.x) {
+        const bool whole = i < full;
+        if (!whole && j >= a0.rem) return;
+        ws_item<S1, S2>(a0, t, whole ? full - 1 - i : full + j,  // the last items (the longest) first
+                        whole ? 0 : c * a0.beta / a0.kch, whole ? a0.beta : (c + 1) * a0.beta / a0.kch,
+                        whole ? nullptr : a0.partial + ((size_t)j * a0.kch + c) * PS, lds, tws);
+        if (!whole) break;
+        __syncthreads();
+    }
     // the chunk's sums are in L2 before its arrival is counted
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -806,23 +1009,17 @@ __device__ __forceinline__ void epi_item(const EpiRows &a, const NttTables &t, c
     T x[SB::E];
 #pragma unroll
     for (int e = 0; e < SB::E; e++) x[e] = ar.load_mid(ld_stream(&a.inter[lo + SB::T * e]));
-    if constexpr (A::kF64) {
-        // stage this item's rows' base factors rb[g][tile ROWS + i] and the
-        // small table in LDS (requested after the residues, so the one wait
-        // covers both) instead of dependent global reads inside the rounds
+    {
+        // stage this item's rows' twiddle factors in LDS (requested after the
+        // residues, so the one wait covers both) instead of dependent global
+        // reads inside the rounds
         using FG = FGeo<S1, S2>;
-        constexpr int RB = S2 * FG::ROWS, NS = RB + (1 << (S2 - 1));
-        const uint32_t tile0 = k1 - k1 % FG::ROWS;
-        const ulonglong2 *rb = t.rb_fw + (size_t)j * S2 * G::N1 + tile0;
-        const ulonglong2 *small = t.small_fw + (size_t)j * kSmall;
-        TwStage<NS, FG::THREADS> st;
-        st.load([&](uint32_t i) { return i < (uint32_t)RB ? rb[(i / FG::ROWS) * G::N1 + i % FG::ROWS] : small[i - RB]; });
-        st.store(twl);
+        using RS = RowStage<S1, S2, FG::ROWS>;
+        RS st;
+        st.load(t, j, k1 / FG::ROWS, true, (uint64_t)ar.q);
+        st.st.store(twl);
         __syncthreads();
-        const TileTw w{nullptr, nullptr, twl, twl + RB, k1 % FG::ROWS};
-        fwd_rows_core<A, S1, S2, FG::ROWS>(x, ar, w, k1, lr);
-    } else {
-        fwd_rows_core<A, S1, S2>(x, ar, t, j, k1, lr);
+        fwd_rows_core<A, S1, S2, FG::ROWS>(x, ar, RS::view(twl, t.tw + (size_t)j * G::N, k1 % FG::ROWS), k1, lr);
     }
     const uint64_t *cp = a.c + m * a.c_stride + (size_t)j * G::N + rowoff;
     const uint64_t *bp = (m & 1u) ? a.base1 : a.base0;
@@ -856,9 +1053,9 @@ __device__ __forceinline__ void epi_item(const EpiRows &a, const NttTables &t, c
                     ar.mul(d, f);
                     v = ar.store(d);
                 } else {
-                    const uint64_t cf = shoup(cv[i], f1.x, f1.y, ar.q);
-                    const uint64_t d = sub_mod(add_mod(cf, bv[i], ar.q), ar.store(x[e]), ar.q);
-                    v = shoup(d, f.x, f.y, ar.q);
+                    // within (1.6 + 0.6) q, then the base in [0, q)
+                    ar.reduce(x[e]);
+                    v = ar.store(ar.mulw(ar.mulw(cv[i], f1) - x[e] + bv[i], f));
                 }
             } else if constexpr (A::kF64) {
                 ar.reduce(x[e]);
@@ -867,9 +1064,8 @@ __device__ __forceinline__ void epi_item(const EpiRows &a, const NttTables &t, c
                 v = ar.store(d);
                 if (bp) v = add_mod(v, bv[i], (uint64_t)ar.q);
             } else {
-                const uint64_t d = sub_mod(cv[i], ar.store(x[e]), ar.q);
-                v = shoup(d, f.x, f.y, ar.q);
-                if (bp) v = add_mod(v, bv[i], ar.q);
+                ar.reduce(x[e]);
+                v = ar.store(ar.mulw(cv[i] - x[e], f) + bv[i]);
             }
             st_stream(&op[SB::T * e], v);
         }
@@ -877,12 +1073,12 @@ __device__ __forceinline__ void epi_item(const EpiRows &a, const NttTables &t, c
 }
 
 template <int S1, int S2>
-__global__ void __launch_bounds__((FGeo<S1, S2>::THREADS))
+__global__ void __launch_bounds__((FGeo<S1, S2>::THREADS)) __attribute__((amdgpu_waves_per_eu(S2 == 8 ? 4 : 3, 8)))
 k_epi_rows(EpiRows a, NttTables t) {
     using G = Geo<S1, S2>;
     using FG = FGeo<S1, S2>;
     __shared__ double lds[FG::LDS];
-    __shared__ ulonglong2 twl[S2 * FG::ROWS + (1 << (S2 - 1))];
+    __shared__ ulonglong2 twl[RowStage<S1, S2, FG::ROWS>::N];
     const uint32_t rr = threadIdx.x / Sub<S2>::T;
     const uint32_t total = a.M * a.J * FG::TILES;
     for (uint32_t p = blockIdx.x; p < total; p += gridDim.x) {
@@ -908,16 +1104,19 @@ k_epi_rows(EpiRows a, NttTables t) {
 // limb.  128-bit products, one Barrett reduction (alpha < 64 keeps the sum
 // below 2^128 for residues below 2^61).
 __global__ void k_mdr_last(uint64_t *x, const uint64_t *g, const uint64_t *mod, const ulonglong2 *ratio,
-                           uint32_t row, uint32_t alpha, uint32_t N, uint32_t M) {
+                           uint32_t row, uint32_t Q, uint32_t alpha, uint32_t N, uint32_t M, uint32_t split30) {
     const uint64_t q = mod[row];
     const ulonglong2 rt = ratio[row];
+    // 30-bit halves (limbs of primes of 50 bits or more when split30 is set)
+    const auto join = [](uint64_t v) { return (v >> 32 << 30) + (uint32_t)v; };
+    const bool split0 = split30 && q >= kF64PrimeBound;
     const uint32_t total = M * N;
     for (uint32_t idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += gridDim.x * blockDim.x) {
         const uint32_t m = idx / N, k = idx % N;
         uint64_t *base = x + (size_t)m * (alpha + 1) * N + k;
         // the limbs' values are requested before the first product, 8 at a time
         // (a rolled loop waited for each value before requesting the next)
-        const uint64_t x0 = base[0];
+        const uint64_t x0 = split0 ? join(base[0]) : base[0];
         U128 acc{0, 0};
         for (uint32_t i0 = 0; i0 < alpha; i0 += 8) {
             uint64_t v[8];
@@ -926,9 +1125,12 @@ __global__ void k_mdr_last(uint64_t *x, const uint64_t *g, const uint64_t *mod, 
                 if (i0 + u < alpha) v[u] = base[(size_t)(i0 + u + 1) * N];
 #pragma unroll
             for (uint32_t u = 0; u < 8; u++)
-                if (i0 + u < alpha) mac(acc, v[u], ld_const(g + i0 + u));
+                if (i0 + u < alpha)
+                    mac(acc, split30 && ld_const(mod + Q + i0 + u) >= kF64PrimeBound ? join(v[u]) : v[u],
+                        ld_const(g + i0 + u));
         }
-        base[0] = sub_mod(x0, barrett128(acc, q, rt.x, rt.y), q);
+        const uint64_t r = sub_mod(x0, barrett128(acc, q, rt.x, rt.y), q);
+        base[0] = split0 ? ((r >> 30) << 32) | ((uint32_t)r & ((1u << 30) - 1)) : r;
     }
 }
 
@@ -1010,7 +1212,7 @@ __device__ __forceinline__ void tensor_rows_tile(const TensorRows &a, RowStage<S
         }
     }
     __syncthreads();
-    const TileTw w = RS::view(twl, a.itw, threadIdx.x / Sub<S2>::T);
+    const StagedTw w = RS::view(twl, a.itw, threadIdx.x / Sub<S2>::T);
     inv_rows_lds<A, S1, S2, R, true, R>(w, r, q, lds, a.mid + r.m * a.mid_stride + (size_t)r.l * G::N,
                                         threadIdx.x < NR);
 }
@@ -1028,7 +1230,7 @@ k_tensor_rows(TensorRows a, NttTables t) {
     a.itw = t.itw + (size_t)r.l * G::N;
     // the tile's twiddle factors are requested before its residues
     RS stage;
-    stage.load(t, r.l, r.tile, false);
+    stage.load(t, r.l, r.tile, false, q);
     if (q < kF64PrimeBound)
         tensor_rows_tile<ArithF64, S1, S2, R, MT>(a, stage, twl, r, q, lds);
     else
@@ -1045,17 +1247,29 @@ uint32_t fgrid(const Ctx &c, uint32_t items, uint32_t wpc) {
     return items < cap ? items : cap;
 }
 
+// whether base conversions of up to n inputs may sum 30-bit limbs
+bool limb_sums(const Ctx &c, uint32_t n) { return c.max_modulus < (1ull << 60) && n <= kLimbInputs; }
+
 template <int S1, int S2>
 void launch_bconv(const Ctx &c, const BconvCols &a0, hipStream_t s) {
     using G = Geo<S1, S2>;
     BconvCols a = a0;
-    // the Montgomery-accumulated sums need sum_i t_i < 2^64; every input is
-    // below the context's largest prime
-    if (c.max_modulus <= ~0ull / std::max(a.n_in, a.n_in_last)) a.mont = c.mont;
+    // every input is below the context's largest prime
+    a.mont = c.mont;
+    a.sum128 = c.max_modulus <= ~0ull / std::max(a.n_in, a.n_in_last);
     const uint32_t total = grouped_total(a.batch * a.groups * G::COL_TILES, a.J);
     const uint32_t grid = fgrid(c, total, 4);
     if (a.sched && (grid != a.sched_grid || total != a.sched_total)) a.sched = nullptr;
-    hipLaunchKernelGGL((k_bconv_cols<S1, S2>), dim3(grid), dim3(G::COL_THREADS), 0, s, a, tables_of(c));
+    const uint32_t n = std::max(a.n_in, a.n_in_last);
+    const auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(G::COL_THREADS), 0, s, a, tables_of(c));
+    };
+    if (n == 1)
+        go(k_bconv_cols<S1, S2, kOne>);
+    else if (limb_sums(c, n))
+        go(k_bconv_cols<S1, S2, kLimbs>);
+    else
+        go(k_bconv_cols<S1, S2, kWide>);
     PFA_HIP(hipGetLastError());
 }
 
@@ -1177,13 +1391,17 @@ static void modup_cols(const Ctx &c, uint32_t chain, const uint64_t *c2, uint64_
     const uint64_t LN = (uint64_t)Ql * c.N, IN = (uint64_t)lv.beta * QlP * c.N;
     Scratch sc(c, s);
     uint64_t *tin = sc.alloc((size_t)batch * LN);
+    // with more than one input a digit the INTT leaves wide residues split
+    const bool split30 = alpha > 1 && limb_sums(c, alpha);
     if (c2_mid) {
         NttLaunch inv{c2_mid, tin, LN, LN, batch, Ql};
         inv.scale = lv.modup_scale;
+        inv.split30 = split30;
         ntt_inverse_cols(c, inv, s);
     } else {
         NttLaunch inv{c2, tin, c2_stride, LN, batch, Ql};
         inv.scale = lv.modup_scale;
+        inv.split30 = split30;
         ntt_inverse(c, inv, s);
     }
     BconvCols b{};
@@ -1204,6 +1422,7 @@ static void modup_cols(const Ctx &c, uint32_t chain, const uint64_t *c2, uint64_
     b.bc_gstride = 2 * alpha * QlP;
     b.bc_istride = QlP;
     b.unit = alpha == 1;
+    b.split30 = split30;
     b.batch = batch;
     b.in_bstride = LN;
     b.out_bstride = IN;
@@ -1311,7 +1530,7 @@ k_galois_rows(GaloisRows a, NttTables t) {
     const uint64_t *src = a.src + i * a.src_stride + row;
     uint64_t *dst = a.dst + (size_t)i * 2 * a.Ql * G::N + row + tb;
     RS stage;
-    if (k) stage.load(t, r.l, r.tile, false);  // requested before the residues
+    if (k) stage.load(t, r.l, r.tile, false, q);  // requested before the residues
     uint64_t v[E];
 #pragma unroll
     for (uint32_t p = 0; p < E; p++) v[p] = src[galois_perm(e, tb + threadIdx.x + NT * p, a.logN)];
@@ -1328,7 +1547,7 @@ k_galois_rows(GaloisRows a, NttTables t) {
     // the staged twiddles were requested first: this waits for them only
     stage.st.store(twl);
     uint64_t *mid = a.mid + ((size_t)i * a.Ql + r.l) * G::N;
-    const TileTw w = RS::view(twl, t.itw + (size_t)r.l * G::N, threadIdx.x / Sub<S2>::T);
+    const StagedTw w = RS::view(twl, t.itw + (size_t)r.l * G::N, threadIdx.x / Sub<S2>::T);
     if (q < kF64PrimeBound) {
         const ArithF64 ar(q);
 #pragma unroll
@@ -1398,9 +1617,10 @@ void fused_moddown_rescale(const Ctx &c, uint32_t chain, const uint64_t *cx, con
     inv.split = 1;
     inv.split_base = c.Q;
     inv.scale = lv.mdr_scale;
+    inv.split30 = limb_sums(c, alpha + 1);
     ntt_inverse(c, inv, s);
     hipLaunchKernelGGL(k_mdr_last, dim3((M * c.N + 255) / 256), dim3(256), 0, s, x, lv.mdr_glast, c.mod, c.ratio,
-                       Ql - 1, alpha, c.N, M);
+                       Ql - 1, c.Q, alpha, c.N, M, inv.split30 ? 1u : 0u);
     PFA_HIP(hipGetLastError());
     BconvCols b{};
     b.in = x;
@@ -1415,6 +1635,7 @@ void fused_moddown_rescale(const Ctx &c, uint32_t chain, const uint64_t *cx, con
     b.in_row0 = c.Q;
     b.in_row_step = 0;
     b.first_row = Ql - 1;
+    b.split30 = inv.split30;
     b.split = 0xffffffffu;
     b.split_base = 0;
     b.skip = 0;
@@ -1438,8 +1659,10 @@ void fused_moddown(const Ctx &c, uint32_t chain, const uint64_t *cx, uint32_t M,
     NttLaunch inv{cx + (size_t)Ql * c.N, xP, (uint64_t)QlP * c.N, (uint64_t)alpha * c.N, M, alpha};
     inv.start = c.Q;
     inv.scale = c.moddown_scale;
+    inv.split30 = alpha > 1 && limb_sums(c, alpha);
     ntt_inverse(c, inv, s);
     BconvCols b{};
+    b.split30 = inv.split30;
     b.in = xP;
     b.out = inter;
     b.bc = c.moddown_bc;

@@ -59,7 +59,7 @@ inline uint64_t shoup_of(uint64_t w, uint64_t q) { return (uint64_t)(((u128)w <<
 bool is_prime(uint64_t n);
 uint64_t minimal_root(uint64_t degree, uint64_t q);
 // Pair encoding of a constant w mod q for the NTT arithmetic policy of q
-// (integer Shoup pair, or (double w, fl(w/q)) for q < 2^50).
+// ((double w, fl(w/q)) for q < 2^50, else ArithInt's centred pair).
 ulonglong2 ntt_pair(uint64_t w, uint64_t q);
 // Integer Shoup pair (w, floor(w 2^64/q)) for the elementwise kernels.
 inline ulonglong2 shoup_pair(uint64_t w, uint64_t q) { return ulonglong2{w, shoup_of(w, q)}; }
@@ -76,8 +76,8 @@ struct Level {
     uint64_t *modup_mat = nullptr;
     // rescale: [q_last^-1]_{q_j} Shoup pairs, j < Ql - 1
     ulonglong2 *rescale_inv = nullptr;
-    // fused path: modup_mat entries as NTT-policy pairs of the target prime,
-    // [beta][alpha][QlP][2] = (m, [m 2^32]_{p_r}); rescale factor as NTT pairs
+    // fused path: modup_mat entries m for the target prime p_r,
+    // [beta][alpha][QlP][2] = (NTT pair of m, bconv_pair1); rescale factor as NTT pairs
     ulonglong2 *modup_bc = nullptr;
     ulonglong2 *rescale_inv_p = nullptr;
     // fused ModDown + rescale, with q_l = this level's last prime:
@@ -188,14 +188,13 @@ struct Ctx {
     ulonglong2 *moddown_scale = nullptr;
     uint64_t *moddown_mat = nullptr;
     ulonglong2 *pinv = nullptr;
-    // fused path: moddown_mat as NTT-policy pairs [P][Q][2] = (m, [m 2^32]_{q_i}),
-    // (1, [2^32]_{q_i}) per Q prime [Q][2], [P^-1]_{q_i} as NTT-policy pairs [Q]
+    // fused path: moddown_mat [P][Q][2] in modup_bc's form, the factor 1 per Q
+    // prime [Q][2], [P^-1]_{q_i} as NTT-policy pairs [Q]
     ulonglong2 *moddown_bc = nullptr;
     ulonglong2 *unit_bc = nullptr;
     ulonglong2 *pinv_p = nullptr;
     // fused ModDown + rescale base conversion [1 + P][Q][2]: input 0 (the
-    // rescale's last limb) with (1, [2^32]_{q_i}), input 1 + j with
-    // ([p_j^-1]_{q_i}, [p_j^-1 2^32]_{q_i}), NTT-policy pairs
+    // rescale's last limb) with factor 1, input 1 + j with [p_j^-1]_{q_i}
     ulonglong2 *mdr_bc = nullptr;
     // key construction: [P]_{q_i} Shoup pairs over all QP rows (0 on P rows)
     ulonglong2 *pmodq = nullptr;
@@ -307,6 +306,9 @@ struct NttLaunch {
     uint32_t start = 0, split = 0xffffffffu, split_base = 0;
     uint32_t ex_lo = 0, ex_step = 0, ex_len = 0, ex_cap = 0;
     const ulonglong2 *scale = nullptr;
+    // inverse only: limbs of primes of 50 bits or more leave as 30-bit halves,
+    // (v >> 30) 2^32 + (v mod 2^30), the form the base conversions multiply
+    bool split30 = false;
 };
 // allow_flow false keeps the transform on the two-launch path, which needs no
 // workspace (the single-launch path takes control blocks from it)

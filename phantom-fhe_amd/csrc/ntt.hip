@@ -24,6 +24,7 @@ NttBatch make_batch(const Ctx &c, const NttLaunch &a) {
     b.ex_len = a.ex_len;
     b.ex_cap = a.ex_cap;
     b.scale = a.scale;
+    b.split30 = a.split30;
     return b;
 }
 

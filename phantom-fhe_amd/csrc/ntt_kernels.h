@@ -47,6 +47,7 @@ struct NttBatch {
     uint32_t ex_lo, ex_step, ex_len, ex_cap;
     // optional per-limb scale applied after the inverse (pair table indexed by l)
     const ulonglong2 *scale;
+    bool split30;  // inverse: integer-policy limbs leave as 30-bit halves (NttLaunch)
     __device__ __forceinline__ bool excluded(uint32_t m, uint32_t l) const {
         uint32_t lo = ex_lo + m * ex_step;
         uint32_t hi = lo + ex_len;
@@ -84,6 +85,69 @@ struct Sub {
 };
 
 // ---------------------------------------------------------------- rounds
+// Before stage number i of a forward integer round (the FP64 policy's four
+// stages need none): see the bounds in modarith.h.
+template <class A, int E>
+__device__ __forceinline__ void fwd_guard(typename A::T (&x)[E], const A &ar, int i) {
+    if constexpr (!A::kF64) {
+        if (i == 0) return;
+        if (i % 4 == 0 || ar.tight) {
+#pragma unroll
+            for (int e = 0; e < E; e++) ar.reduce(x[e]);
+        }
+    }
+}
+
+// Which of the E elements of an inverse integer round of NS stages (distances
+// 1, 2, 4, ...) are reduced: before stage i (red[i]) and after the last one
+// (red[NS]).  Bounds are followed in sixteenths of q: a stage of distance d
+// takes the bounds of (e, e + d) to their sum and to 1.5 + an eighth of it; a
+// sum must stay below 8 q, and the round hands on at most 2 q.  b0: the bound
+// it starts from.
+template <int E, int NS>
+struct InvReduce {
+    static constexpr int kRed = 9, kLim = 62, kOut = 32;
+    uint32_t red[NS + 1];
+    constexpr InvReduce(int b0) : red{} {
+        int b[E] = {};
+        for (int e = 0; e < E; e++) b[e] = b0;
+        for (int i = 0; i <= NS; i++) {
+            for (int e = 0; e < E; e++)
+                if (b[e] > (i < NS ? kLim : kOut)) {
+                    red[i] |= 1u << e;
+                    b[e] = kRed;
+                }
+            if (i == NS) break;
+            const int d = 1 << i;
+            for (int e = 0; e < E; e++)
+                if (!(e & d)) {
+                    const int s = b[e] + b[e + d];
+                    b[e] = s;
+                    b[e + d] = 24 + (s + 7) / 8;
+                }
+        }
+    }
+};
+
+// Reductions of InvReduce before stage I of an inverse round (I = NS: after
+// it).  With values of 4 q only (tight) every element is reduced.
+template <class A, int E, int NS, int B0, int I>
+__device__ __forceinline__ void inv_guard(typename A::T (&x)[E], const A &ar) {
+    if constexpr (!A::kF64) {
+        constexpr uint32_t mask = InvReduce<E, NS>(B0).red[I];
+        // keeps a stage's twiddle reads behind the stage before it (registers)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int e = 0; e < E; e++)
+            if ((mask >> e) & 1u) ar.reduce(x[e]);
+        if (I > 0 && ar.tight) {
+#pragma unroll
+            for (int e = 0; e < E; e++)
+                if (!((mask >> e) & 1u)) ar.reduce(x[e]);
+        }
+    }
+}
+
 // forward, stages g = 0 .. LE-1 on elements u = F + T e
 template <class A, int S>
 __device__ __forceinline__ void fwd_round_a(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
@@ -92,6 +156,7 @@ __device__ __forceinline__ void fwd_round_a(typename A::T (&x)[Sub<S>::E], const
 #pragma unroll
     for (int g = 0; g < LE; g++) {
         const int d = E >> (g + 1);
+        fwd_guard(x, ar, g);
 #pragma unroll
         for (int e = 0; e < E; e++) {
             if (e & d) continue;
@@ -109,6 +174,7 @@ __device__ __forceinline__ void fwd_round_b(typename A::T (&x)[Sub<S>::E], const
     for (int g = LE; g < S; g++) {
         const int d = 1 << (S - 1 - g);
         const ulonglong2 *t = tw + (base << g) + (F << (LE - S + g));
+        fwd_guard(x, ar, g - LE);
 #pragma unroll
         for (int e = 0; e < E; e++) {
             if (e & d) continue;
@@ -117,32 +183,36 @@ __device__ __forceinline__ void fwd_round_b(typename A::T (&x)[Sub<S>::E], const
     }
 }
 
-// inverse, stages g = S-1 .. LE on elements u = F' E + e
-template <class A, int S>
+// inverse, stages g = S-1 .. LE on elements u = F' E + e (stage I of the round:
+// g = S-1-I, distance 2^I).  B0: the bound on the elements in sixteenths of q
+// (16: canonical residues; 9: reduced ones).
+template <class A, int S, int B0, int I = 0>
 __device__ __forceinline__ void inv_round_a(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *itw,
                                             uint32_t base, uint32_t F) {
-    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
-#pragma unroll
-    for (int g = S - 1; g >= LE; g--) {
-        const int d = 1 << (S - 1 - g);
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E, G = S - LE, g = S - 1 - I, d = 1 << I;
+    if constexpr (I < G) {
+        inv_guard<A, E, G, B0, I>(x, ar);
         const ulonglong2 *t = itw + (base << g) + (F << (LE - S + g));
 #pragma unroll
         for (int e = 0; e < E; e++) {
             if (e & d) continue;
             ar.gs(x[e], x[e + d], t[e >> (S - g)]);
         }
+        inv_round_a<A, S, B0, I + 1>(x, ar, itw, base, F);
+    } else {
+        inv_guard<A, E, G, B0, G>(x, ar);
     }
 }
 
-// inverse, stages g = LE-1 .. 0 on elements u = F + T e.  With LAST the g = 0
-// stage folds N^-1 into the sum half (the difference half gets it from itw[1]).
-template <class A, int S, bool LAST>
+// inverse, stages g = LE-1 .. 0 on elements u = F + T e (stage I of the round:
+// g = LE-1-I), from a bound of 2 q.  With LAST the g = 0 stage folds N^-1 into
+// the sum half (the difference half gets it from itw[1]).
+template <class A, int S, bool LAST, int I = 0>
 __device__ __forceinline__ void inv_round_b(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *itw,
                                             uint32_t base, ulonglong2 ninv) {
-    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
-#pragma unroll
-    for (int g = LE - 1; g >= 0; g--) {
-        const int d = E >> (g + 1);
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E, g = LE - 1 - I, d = E >> (g + 1);
+    if constexpr (I < LE) {
+        inv_guard<A, E, LE, 32, I>(x, ar);
 #pragma unroll
         for (int e = 0; e < E; e++) {
             if (e & d) continue;
@@ -151,6 +221,117 @@ __device__ __forceinline__ void inv_round_b(typename A::T (&x)[Sub<S>::E], const
             else
                 ar.gs(x[e], x[e + d], itw[(base << g) + (e >> (LE - g))]);
         }
+        inv_round_b<A, S, LAST, I + 1>(x, ar, itw, base, ninv);
+    }
+}
+
+// Entry i of a table at a wave-uniform base: the byte offset is kept in 32 bits
+// (a table is at most 2 MiB), so the load takes the base from scalar registers
+// and one vector register of offset instead of a 64-bit vector address.
+__device__ __forceinline__ ulonglong2 tw_at(const ulonglong2 *tw, uint32_t i) {
+    return *reinterpret_cast<const ulonglong2 *>(reinterpret_cast<const char *>(tw) + (size_t)(uint32_t)(i * 16u));
+}
+
+// The twiddles one thread uses in a sub-transform's second round (stages LE ..
+// S-1, at its element block F), requested together: a rows pass of the integer
+// policy reads them from the prime's full table, and one load after the other
+// (each stage's after the stage before it) leaves the L2's latency exposed at
+// every stage.
+template <int S>
+struct TwB {
+    static constexpr int LE = Sub<S>::LE, O = 1 << (2 * LE - S), N = (1 << LE) - O;
+    ulonglong2 w[N];
+    __device__ __forceinline__ void load(const ulonglong2 *tw, uint32_t base, uint32_t F) {
+#pragma unroll
+        for (int g = LE; g < S; g++)
+#pragma unroll
+            for (int i = 0; i < (1 << (LE - S + g)); i++)
+                w[(1 << (LE - S + g)) - O + i] = tw_at(tw, (base << g) + (F << (LE - S + g)) + i);
+    }
+    __device__ __forceinline__ ulonglong2 at(int g, int i) const { return w[(1 << (LE - S + g)) - O + i]; }
+};
+
+// First-round entries (stages 0 .. LE-1, the same for every thread of a row)
+// in LDS: entry i of stage g at 2^g - 1 + i.
+struct LdsTwA {
+    const ulonglong2 *w;
+    __device__ __forceinline__ ulonglong2 at(int g, int i) const { return w[(1 << g) - 1 + i]; }
+};
+
+// Second-round entries read from the full table stage by stage (a pass whose
+// registers do not hold TwB).
+template <int S>
+struct TableTwB {
+    static constexpr int LE = Sub<S>::LE;
+    const ulonglong2 *tw;
+    uint32_t base, F;
+    __device__ __forceinline__ ulonglong2 at(int g, int i) const {
+        return tw_at(tw, (base << g) + (F << (LE - S + g)) + i);
+    }
+};
+
+// The integer rounds with their twiddles in W (LdsTwA, TwB, TableTwB)
+template <int S, class W>
+__device__ __forceinline__ void fwd_round_a_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const W &w) {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+#pragma unroll
+    for (int g = 0; g < LE; g++) {
+        const int d = E >> (g + 1);
+        // keeps a stage's twiddle reads behind the stage before it (registers)
+        __builtin_amdgcn_sched_barrier(0);
+        fwd_guard(x, ar, g);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            if (e & d) continue;
+            ar.ct(x[e], x[e + d], w.at(g, e >> (LE - g)));
+        }
+    }
+}
+
+template <int S, class W>
+__device__ __forceinline__ void fwd_round_b_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const W &w) {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+#pragma unroll
+    for (int g = LE; g < S; g++) {
+        const int d = 1 << (S - 1 - g);
+        // keeps a stage's twiddle reads behind the stage before it (registers)
+        __builtin_amdgcn_sched_barrier(0);
+        fwd_guard(x, ar, g - LE);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            if (e & d) continue;
+            ar.ct(x[e], x[e + d], w.at(g, e >> (S - g)));
+        }
+    }
+}
+
+template <int S, int B0, int I = 0>
+__device__ __forceinline__ void inv_round_a_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const TwB<S> &w) {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E, G = S - LE, g = S - 1 - I, d = 1 << I;
+    if constexpr (I < G) {
+        inv_guard<ArithInt, E, G, B0, I>(x, ar);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            if (e & d) continue;
+            ar.gs(x[e], x[e + d], w.at(g, e >> (S - g)));
+        }
+        inv_round_a_int<S, B0, I + 1>(x, ar, w);
+    } else {
+        inv_guard<ArithInt, E, G, B0, G>(x, ar);
+    }
+}
+
+template <int S, int I = 0, class W>
+__device__ __forceinline__ void inv_round_b_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const W &w) {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E, g = LE - 1 - I, d = E >> (g + 1);
+    if constexpr (I < LE) {
+        inv_guard<ArithInt, E, LE, 32, I>(x, ar);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            if (e & d) continue;
+            ar.gs(x[e], x[e + d], w.at(g, e >> (LE - g)));
+        }
+        inv_round_b_int<S, I + 1>(x, ar, w);
     }
 }
 
@@ -370,6 +551,14 @@ struct TileTw {
     const ulonglong2 *rb;
     const ulonglong2 *small;
     uint32_t rrow;
+    static constexpr bool kStaged = false;
+};
+
+// The same with the factors in LDS: rb and small point there, and ra at the
+// row's first-round entries (LdsTwA, integer policy).
+struct StagedTw : TileTw {
+    const ulonglong2 *ra;
+    static constexpr bool kStaged = true;
 };
 
 template <int S1, int S2>
@@ -408,23 +597,36 @@ struct TwStage {
     }
 };
 
-// Staged entries of a rows-pass tile: rb[g][tile ROWS + i] for g < S2, i < ROWS,
-// then the small table's first 2^(S2-1) entries.
+// Staged entries of a rows-pass tile.  FP64 policy: rb[g][tile R + i] for
+// g < S2, i < R, then the small table's first 2^(S2-1) entries; integer policy:
+// the first-round entries (LdsTwA) of the R rows, E slots a row.
 template <int S1, int S2, int R = Geo<S1, S2>::ROWS>
 struct RowStage {
     using G = Geo<S1, S2>;
-    static constexpr int RB = S2 * R;
-    static constexpr int N = RB + (1 << (S2 - 1));
+    static constexpr int RB = S2 * R, E = Sub<S2>::E;
+    static constexpr int NF = RB + (1 << (S2 - 1)), NI = R * E;
+    static constexpr int N = NF > NI ? NF : NI;
     TwStage<N, R * Sub<S2>::T> st;
-    __device__ __forceinline__ void load(const NttTables &t, uint32_t prow, uint32_t tile, bool fwd) {
-        const ulonglong2 *rb = (fwd ? t.rb_fw : t.rb_inv) + (size_t)prow * S2 * G::N1 + tile * R;
-        const ulonglong2 *small = (fwd ? t.small_fw : t.small_inv) + (size_t)prow * kSmall;
-        st.load([&](uint32_t i) { return i < (uint32_t)RB ? rb[(i / R) * G::N1 + i % R] : small[i - RB]; });
+    __device__ __forceinline__ void load(const NttTables &t, uint32_t prow, uint32_t tile, bool fwd, uint64_t q) {
+        if (q < kF64PrimeBound) {
+            const ulonglong2 *rb = (fwd ? t.rb_fw : t.rb_inv) + (size_t)prow * S2 * G::N1 + tile * R;
+            const ulonglong2 *small = (fwd ? t.small_fw : t.small_inv) + (size_t)prow * kSmall;
+            st.load([&](uint32_t i) {
+                return i < (uint32_t)RB ? rb[(i / R) * G::N1 + i % R] : small[i < (uint32_t)NF ? i - RB : 0];
+            });
+        } else {
+            const ulonglong2 *tab = (fwd ? t.tw : t.itw) + (size_t)prow * G::N;
+            st.load([&](uint32_t i) {
+                const uint32_t j = i < (uint32_t)NI ? i % E : 0, row = i < (uint32_t)NI ? i / E : 0;
+                const uint32_t e = j < (uint32_t)E - 1 ? j : 0, g = 31 - __builtin_clz(e + 1);
+                return tab[((G::N1 + tile * R + row) << g) + (e + 1 - (1u << g))];
+            });
+        }
     }
     // LDS copy -> the tile's twiddle view (full: the prime's global table, for
-    // the integer policy)
-    __device__ __forceinline__ static TileTw view(const ulonglong2 *lds, const ulonglong2 *full, uint32_t rr) {
-        return TileTw{nullptr, full, lds, lds + RB, rr};
+    // the integer policy's second round)
+    __device__ __forceinline__ static StagedTw view(const ulonglong2 *lds, const ulonglong2 *full, uint32_t rr) {
+        return StagedTw{{nullptr, full, lds, lds + RB, rr}, lds + rr * E};
     }
 };
 
@@ -443,9 +645,9 @@ __device__ __forceinline__ const uint64_t *cols_src(const NttBatch &b, const Til
 // table (entries 1 .. N1-1 are read).
 template <class A, int S1, int S2>
 __device__ __forceinline__ void fwd_cols_core(typename A::T (&x)[Sub<S1>::E], const A &ar, const ulonglong2 *tw,
-                                              typename A::T *lds) {
+                                              typename A::T *lds, uint32_t tid = threadIdx.x) {
     using SB = Sub<S1>;
-    const uint32_t c = threadIdx.x % kCols, F = threadIdx.x / kCols;
+    const uint32_t c = tid % kCols, F = tid / kCols;
     fwd_round_a<A, S1>(x, ar, tw, 1);
 #pragma unroll
     for (int e = 0; e < SB::E; e++) {
@@ -463,11 +665,11 @@ __device__ __forceinline__ void fwd_cols_core(typename A::T (&x)[Sub<S1>::E], co
 // in the same launch)
 template <class A, int S1, int S2, bool NT = true>
 __device__ __forceinline__ void fwd_cols_store(const typename A::T (&x)[Sub<S1>::E], const A &ar, uint32_t tile,
-                                               uint64_t *olimb) {
+                                               uint64_t *olimb, uint32_t tid = threadIdx.x) {
     using G = Geo<S1, S2>;
     using SB = Sub<S1>;
     uint64_t *dst = olimb + tile * kCols;
-    const uint32_t c = threadIdx.x % kCols, F = threadIdx.x / kCols;
+    const uint32_t c = tid % kCols, F = tid / kCols;
 #pragma unroll
     for (int e = 0; e < SB::E; e++) {
         uint64_t *p = &dst[(size_t)(F * SB::E + e) * G::N2 + c];
@@ -536,14 +738,16 @@ ntt_fwd_cols(NttBatch b, NttTables t) {
 // row in the intermediate form.  Out: x[e] = element (F + T e) of the
 // transformed row (lazy; the final LDS transpose makes stores coalesced).
 // The caller separates consecutive calls on the same LDS with a barrier.
-template <class A, int S1, int S2, int RBS>
-__device__ __forceinline__ void fwd_rows_core(typename A::T (&x)[Sub<S2>::E], const A &ar, const TileTw &w,
+template <class A, int S1, int S2, int RBS, class TW>
+__device__ __forceinline__ void fwd_rows_core(typename A::T (&x)[Sub<S2>::E], const A &ar, const TW &w,
                                               uint32_t k1, typename A::T *lr) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
     const uint32_t F = threadIdx.x % SB::T;
     if constexpr (A::kF64)
         fwd_round_a_derived<S2, RBS>(x, ar, w.rb, w.small, w.rrow);
+    else if constexpr (TW::kStaged)
+        fwd_round_a_int<S2>(x, ar, LdsTwA{w.ra});
     else
         fwd_round_a<A, S2>(x, ar, w.full, G::N1 + k1);
 #pragma unroll
@@ -556,6 +760,8 @@ __device__ __forceinline__ void fwd_rows_core(typename A::T (&x)[Sub<S2>::E], co
     for (int e = 0; e < SB::E; e++) x[e] = lr[rpad(F * SB::E + e)];
     if constexpr (A::kF64)
         fwd_round_b_derived<S2, RBS>(x, ar, w.rb, w.small, w.rrow, F);
+    else if constexpr (TW::kStaged)
+        fwd_round_b_int<S2>(x, ar, TableTwB<S2>{w.full, G::N1 + k1, F});
     else
         fwd_round_b<A, S2>(x, ar, w.full, G::N1 + k1, F);
     __syncthreads();
@@ -573,8 +779,8 @@ __device__ __forceinline__ void fwd_rows_core(typename A::T (&x)[Sub<S2>::E], co
     fwd_rows_core<A, S1, S2, Geo<S1, S2>::N1>(x, ar, global_tw<S1, S2>(t, prow, k1, true), k1, lr);
 }
 
-template <class A, int S1, int S2, int RBS, int R = Geo<S1, S2>::ROWS>
-__device__ __forceinline__ void fwd_rows_tile(const uint64_t (&raw)[Sub<S2>::E], const TileTw &w, const TileRef &r,
+template <class A, int S1, int S2, int RBS, int R = Geo<S1, S2>::ROWS, class TW>
+__device__ __forceinline__ void fwd_rows_tile(const uint64_t (&raw)[Sub<S2>::E], const TW &w, const TileRef &r,
                                               uint64_t q, typename A::T *lds, uint64_t *olimb) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
@@ -614,18 +820,18 @@ ntt_fwd_rows(NttBatch b, NttTables t) {
          cur = next_tile(b, TILES, cur + gridDim.x, total)) {
         const TileRef r = decode_tile(b, TILES, cur);
         const uint32_t prow = b.map.row(r.l);
-        const uint64_t q = t.mod[prow];
+        const uint64_t q = ld_const(t.mod + prow);
         // the tile's twiddles are requested before its residues, so both are
         // in flight together and staged in LDS once
         RS stage;
-        stage.load(t, prow, r.tile, true);
+        stage.load(t, prow, r.tile, true, q);
         uint64_t raw[SB::E];
         const uint64_t *s = rows_ptr<S1, S2, R>(b, r, b.src, b.sstride);
 #pragma unroll
         for (int e = 0; e < SB::E; e++) raw[e] = ld_stream(&s[F + SB::T * e]);
         stage.st.store(twl);
         __syncthreads();
-        const TileTw w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
+        const StagedTw w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
         uint64_t *olimb = b.dst + r.m * b.dstride + (size_t)r.l * G::N;
         if (q < kF64PrimeBound)
             fwd_rows_tile<ArithF64, S1, S2, R, R>(raw, w, r, q, lds, olimb);
@@ -641,8 +847,8 @@ ntt_fwd_rows(NttBatch b, NttTables t) {
 // rr at lds[rr ROW_PITCH + rpad(k)], as A::load gives it), after a barrier.
 // With active false (whole waves beyond the tile's R T threads of a larger
 // workgroup) a thread only takes part in the barriers.
-template <class A, int S1, int S2, int RBS, bool NT = true, int R = Geo<S1, S2>::ROWS>
-__device__ __forceinline__ void inv_rows_lds(const TileTw &w, const TileRef &r, uint64_t q, typename A::T *lds,
+template <class A, int S1, int S2, int RBS, bool NT = true, int R = Geo<S1, S2>::ROWS, class TW>
+__device__ __forceinline__ void inv_rows_lds(const TW &w, const TileRef &r, uint64_t q, typename A::T *lds,
                                              uint64_t *olimb, bool active = true) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
@@ -653,13 +859,21 @@ __device__ __forceinline__ void inv_rows_lds(const TileTw &w, const TileRef &r, 
     uint64_t *drow = olimb + (size_t)k1 * G::N2;
     T *lr = lds + rr * G::ROW_PITCH;
     T x[SB::E];
+    // integer twiddles: the second round's (this one's first) requested
+    // together, the first round's from LDS
+    constexpr bool PRE = !A::kF64 && TW::kStaged && SB::LE <= 4;
     if (active) {
 #pragma unroll
         for (int e = 0; e < SB::E; e++) x[e] = lr[rpad(F * SB::E + e)];
-        if constexpr (A::kF64)
+        if constexpr (A::kF64) {
             inv_round_a_derived<S2, RBS>(x, ar, w.rb, w.small, w.rrow, F);
-        else
-            inv_round_a<A, S2>(x, ar, w.full, G::N1 + k1, F);
+        } else if constexpr (PRE) {
+            TwB<S2> wb;
+            wb.load(w.full, G::N1 + k1, F);
+            inv_round_a_int<S2, 16>(x, ar, wb);
+        } else {
+            inv_round_a<A, S2, 16>(x, ar, w.full, G::N1 + k1, F);
+        }
     }
     __syncthreads();
     if (active) {
@@ -672,6 +886,8 @@ __device__ __forceinline__ void inv_rows_lds(const TileTw &w, const TileRef &r, 
     for (int e = 0; e < SB::E; e++) x[e] = lr[rpad(F + SB::T * e)];
     if constexpr (A::kF64)
         inv_round_b_derived<S2, RBS>(x, ar, w.rb, w.small, w.rrow);
+    else if constexpr (PRE)
+        inv_round_b_int<S2>(x, ar, LdsTwA{w.ra});
     else
         inv_round_b<A, S2, false>(x, ar, w.full, G::N1 + k1, ulonglong2{0, 0});
 #pragma unroll
@@ -683,8 +899,8 @@ __device__ __forceinline__ void inv_rows_lds(const TileTw &w, const TileRef &r, 
     }
 }
 
-template <class A, int S1, int S2, int RBS, bool NT = true, int R = Geo<S1, S2>::ROWS>
-__device__ __forceinline__ void inv_rows_tile(const uint64_t (&raw)[Sub<S2>::E], const TileTw &w, const TileRef &r,
+template <class A, int S1, int S2, int RBS, bool NT = true, int R = Geo<S1, S2>::ROWS, class TW>
+__device__ __forceinline__ void inv_rows_tile(const uint64_t (&raw)[Sub<S2>::E], const TW &w, const TileRef &r,
                                               uint64_t q, typename A::T *lds, uint64_t *olimb) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
@@ -757,16 +973,16 @@ ntt_inv_rows_staged(NttBatch b, NttTables t) {
          cur = next_tile(b, TILES, cur + gridDim.x, total)) {
         const TileRef r = decode_tile(b, TILES, cur);
         const uint32_t prow = b.map.row(r.l);
-        const uint64_t q = t.mod[prow];
+        const uint64_t q = ld_const(t.mod + prow);
         RS stage;
-        stage.load(t, prow, r.tile, false);
+        stage.load(t, prow, r.tile, false, q);
         uint64_t raw[SB::E];
         const uint64_t *s = rows_ptr<S1, S2, R>(b, r, b.src, b.sstride);
 #pragma unroll
         for (int e = 0; e < SB::E; e++) raw[e] = ld_stream(&s[F + SB::T * e]);
         stage.st.store(twl);
         __syncthreads();
-        const TileTw w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
+        const StagedTw w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
         uint64_t *olimb = b.dst + r.m * b.dstride + (size_t)r.l * G::N;
         if (q < kF64PrimeBound)
             inv_rows_tile<ArithF64, S1, S2, R, true, R>(raw, w, r, q, lds, olimb);
@@ -784,7 +1000,7 @@ ntt_inv_rows_staged(NttBatch b, NttTables t) {
 template <class A, int S1, int S2>
 __device__ __forceinline__ void inv_cols_tile(const uint64_t (&raw)[Sub<S1>::E], const ulonglong2 *itw,
                                               ulonglong2 ninv, const ulonglong2 *scale, const TileRef &r,
-                                              uint64_t q, typename A::T *lds, uint64_t *olimb) {
+                                              uint64_t q, typename A::T *lds, uint64_t *olimb, bool split30) {
     using G = Geo<S1, S2>;
     using SB = Sub<S1>;
     using T = typename A::T;
@@ -794,7 +1010,7 @@ __device__ __forceinline__ void inv_cols_tile(const uint64_t (&raw)[Sub<S1>::E],
     T x[SB::E];
 #pragma unroll
     for (int e = 0; e < SB::E; e++) x[e] = ar.load_mid(raw[e]);
-    inv_round_a<A, S1>(x, ar, itw, 1, F);
+    inv_round_a<A, S1, 9>(x, ar, itw, 1, F);
 #pragma unroll
     for (int e = 0; e < SB::E; e++) lds[(F * SB::E + e) * kColStride + c] = x[e];
     __syncthreads();
@@ -802,12 +1018,17 @@ __device__ __forceinline__ void inv_cols_tile(const uint64_t (&raw)[Sub<S1>::E],
     for (int e = 0; e < SB::E; e++) x[e] = lds[(F + SB::T * e) * kColStride + c];
     inv_round_b<A, S1, true>(x, ar, itw, 1, ninv);
     if (scale) {
-        const ulonglong2 sc = *scale;
+        const ulonglong2 sc = A::kF64 ? *scale : ld_const(scale);
 #pragma unroll
         for (int e = 0; e < SB::E; e++) ar.mul(x[e], sc);
     }
 #pragma unroll
-    for (int e = 0; e < SB::E; e++) st_stream(&data[(size_t)(F + SB::T * e) * G::N2 + c], ar.store(x[e]));
+    for (int e = 0; e < SB::E; e++) {
+        uint64_t v = ar.store(x[e]);
+        if constexpr (!A::kF64)
+            if (split30) v = ((v >> 30) << 32) | ((uint32_t)v & ((1u << 30) - 1));
+        st_stream(&data[(size_t)(F + SB::T * e) * G::N2 + c], v);
+    }
 }
 
 // Like the forward columns pass: no register prefetch (124 VGPRs, 4 waves
@@ -839,10 +1060,10 @@ ntt_inv_cols(NttBatch b, NttTables t) {
         const ulonglong2 *sc = b.scale ? b.scale + r.l : nullptr;
         uint64_t *olimb = b.dst + r.m * b.dstride + (size_t)r.l * G::N;
         if (q < kF64PrimeBound)
-            inv_cols_tile<ArithF64, S1, S2>(raw, twl, t.ninv[prow], sc, r, q, lds, olimb);
+            inv_cols_tile<ArithF64, S1, S2>(raw, twl, t.ninv[prow], sc, r, q, lds, olimb, false);
         else
-            inv_cols_tile<ArithInt, S1, S2>(raw, twl, t.ninv[prow], sc, r, q, reinterpret_cast<uint64_t *>(lds),
-                                            olimb);
+            inv_cols_tile<ArithInt, S1, S2>(raw, twl, ld_const(t.ninv + prow), sc, r, q, reinterpret_cast<uint64_t *>(lds),
+                                            olimb, b.split30);
         __syncthreads();
     }
 }
@@ -1044,14 +1265,14 @@ struct FlowJob {
         } else {
             const uint32_t F = threadIdx.x % S2B::T, rr = threadIdx.x / S2B::T;
             RS stage;
-            stage.load(t, prow, tile, false);
+            stage.load(t, prow, tile, false, q);
             const uint64_t *s = rows_ptr<S1, S2>(b, r, b.src, b.sstride);
             uint64_t raw[S2B::E];
 #pragma unroll
             for (int e = 0; e < S2B::E; e++) raw[e] = ld_stream(&s[F + S2B::T * e]);
             stage.st.store(twl);
             __syncthreads();
-            const TileTw w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
+            const StagedTw w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
             if (q < kF64PrimeBound)
                 inv_rows_tile<ArithF64, S1, S2, G::ROWS, false>(raw, w, r, q, lds, limb);
             else
@@ -1067,14 +1288,14 @@ struct FlowJob {
         if (FWD) {
             const uint32_t F = threadIdx.x % S2B::T, rr = threadIdx.x / S2B::T;
             RS stage;
-            stage.load(t, prow, tile, true);
+            stage.load(t, prow, tile, true, q);
             const uint64_t *s = rows_ptr<S1, S2>(b, r, b.dst, b.dstride);
             uint64_t raw[S2B::E];
 #pragma unroll
             for (int e = 0; e < S2B::E; e++) raw[e] = s[F + S2B::T * e];
             stage.st.store(twl);
             __syncthreads();
-            const TileTw w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
+            const StagedTw w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
             if (q < kF64PrimeBound)
                 fwd_rows_tile<ArithF64, S1, S2, G::ROWS>(raw, w, r, q, lds, limb);
             else
@@ -1091,10 +1312,10 @@ struct FlowJob {
             __syncthreads();
             const ulonglong2 *sc = b.scale ? b.scale + l : nullptr;
             if (q < kF64PrimeBound)
-                inv_cols_tile<ArithF64, S1, S2>(raw, twl, t.ninv[prow], sc, r, q, lds, limb);
+                inv_cols_tile<ArithF64, S1, S2>(raw, twl, t.ninv[prow], sc, r, q, lds, limb, false);
             else
-                inv_cols_tile<ArithInt, S1, S2>(raw, twl, t.ninv[prow], sc, r, q, reinterpret_cast<uint64_t *>(lds),
-                                                limb);
+                inv_cols_tile<ArithInt, S1, S2>(raw, twl, ld_const(t.ninv + prow), sc, r, q, reinterpret_cast<uint64_t *>(lds),
+                                                limb, b.split30);
         }
     }
 };
