@@ -565,6 +565,7 @@ static void destroy(Ctx *c) {
         for (auto &ch : kv.second->chunks) (void)hipFree(ch.base);
         if (kv.second->flow) (void)hipFree(kv.second->flow);
         if (kv.second->ws_counter) (void)hipFree(kv.second->ws_counter);
+        if (kv.second->word) (void)hipHostFree(kv.second->word);
         delete kv.second;
     }
     for (void *p : c->allocations) (void)hipFree(p);

@@ -11,7 +11,7 @@
 //           m_k = round(scale Re z_k), m_(k+N/2) = round(scale Im z_k)
 // (the reference's encode packs coefficients the same way,
 // src/rns_base.cu:49-72).  The DFT is a radix-2 Stockham FFT in double
-// precision, one launch per stage.  A rounded coefficient is reduced into each
+// precision, in two launches that also do the slot order and the twist.  A rounded coefficient is reduced into each
 // prime exactly at any size a double holds (m 2^e with 2^e mod q by squaring,
 // where the reference splits it into 64-bit words, src/rns_base.cu:49-170).
 // Decoding composes each coefficient from all of the plaintext's limbs
@@ -29,31 +29,163 @@ namespace {
 
 constexpr int kThreads = 256;
 
-__global__ void k_enc_scatter(const double2 *values, uint32_t n_values, double2 *W, const uint32_t *perm,
-                              uint32_t M) {
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < M; j += gridDim.x * blockDim.x)
-        W[perm[j]] = j < n_values ? values[j] : double2{0.0, 0.0};
+// The DFT, M = 2^(S1 + S2) points, in two launches.  The radix-2 Stockham
+// network splits by index: its first S1 stages join the 2^S1 points j0 + t B
+// (B = M / 2^S1) of a column j0 and leave them at 2^S1 j0 + w, the other S2
+// join the points k0 + q A (A = 2^S1) and leave them at k0 + A w.  A thread
+// holds 8 points, so three stages are one round in registers, and rounds meet
+// in LDS.  One wave a block (512 points): rounds then cost no wait between
+// waves, and M / 512 blocks spread over the CUs.  Every butterfly multiplies
+// and adds as the stage-by-stage network does, so the results are its own, bit
+// for bit.  Latency bounds it (2^14 points are 256 KB), so what counts is the
+// number of launches: a launch a stage, with its sincospi, took 14 for 2^14
+// points besides one each for the slot order, the twist and the flag.  2^14
+// points: 9.3 + 5.6 us encoding (the first also gathers the slots), 4.2 + 5.4
+// us decoding, against 14 x 2.3 us; whole calls at N = 2^15, host part
+// included: 12 limbs encoded 154 -> 80 us, 3 limbs decoded 426 -> 372 us.
+struct Fft {
+    const double2 *in;
+    double2 *out;
+    const double2 *tw;     // [M / 2] exp(i pi t / (M / 2))
+    const double2 *zeta;   // [M] exp(i pi k / N)
+    const uint32_t *iperm; // [M] the slot of DFT index i
+    uint32_t logm, loga;   // points; stages before this launch
+    double sign;           // of the exponent
+    uint32_t n_values;     // encode: slots given (the others are 0)
+    double scale;          // encode: scale / M
+    uint32_t *bits;        // encode: largest coeff_bits
+};
+
+enum FftEnd { kEncFirst, kEncLast, kDecFirst, kDecLast };
+
+__device__ __forceinline__ void fft2(double2 &a, double2 &b, double2 w, double sign) {
+    const double s = sign * w.y;
+    const double tr = __builtin_fma(b.x, w.x, -(b.y * s));
+    const double ti = __builtin_fma(b.x, s, b.y * w.x);
+    b = double2{a.x - tr, a.y - ti};
+    a = double2{a.x + tr, a.y + ti};
 }
 
-__global__ void k_dec_gather(const double2 *W, double2 *values, const uint32_t *perm, uint32_t M) {
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < M; j += gridDim.x * blockDim.x)
-        values[j] = W[perm[j]];
-}
-
-// One Stockham radix-2 stage of a length-M DFT with kernel exp(sign i 2 pi jk / M);
-// Ns = current sub-transform length.
-__global__ void k_fft_stage(const double2 *in, double2 *out, uint32_t M, uint32_t Ns, double sign) {
-    const uint32_t half = M / 2;
-    for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < half; j += gridDim.x * blockDim.x) {
-        const uint32_t k = j & (Ns - 1);
-        double s, c;
-        sincospi(sign * (double)k / (double)Ns, &s, &c);
-        const double2 a = in[j], b0 = in[j + half];
-        const double2 b{b0.x * c - b0.y * s, b0.x * s + b0.y * c};
-        const uint32_t base = (j - k) * 2 + k;
-        out[base] = double2{a.x + b.x, a.y + b.y};
-        out[base + Ns] = double2{a.x - b.x, a.y - b.y};
+// R stages, the first of sub-transform length ns = 2^ls (in local points), on
+// the points j + u 2^S / 2^R of one column; leaves point j's outputs in order
+// w = 0 .. 2^R - 1 (local index 2^R (j - k) + k + w ns).
+template <int R>
+__device__ __forceinline__ void fft_round(double2 (&x)[1 << R], uint32_t k, uint32_t ls, uint32_t k0, const Fft &f) {
+    double2 y[1 << R];
+#pragma unroll
+    for (int g = 0; g < R; g++) {
+        // x: (u, w), u < 2^(R - g), w < 2^g, at u 2^g + w
+        const int H = 1 << (R - 1 - g), W = 1 << g;
+        const uint32_t shift = f.logm - 1 - f.loga - ls - g;
+#pragma unroll
+        for (int w = 0; w < W; w++) {
+            const uint32_t kl = k + ((uint32_t)w << ls);
+            const double2 t = f.tw[(k0 + (kl << f.loga)) << shift];
+#pragma unroll
+            for (int u = 0; u < H; u++) {
+                double2 a = x[u * W + w], b = x[(u + H) * W + w];
+                fft2(a, b, t, f.sign);
+                y[u * 2 * W + w] = a;
+                y[u * 2 * W + w + W] = b;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < (1 << R); i++) x[i] = y[i];
     }
+}
+
+__device__ __forceinline__ uint32_t coeff_bits(double v);
+
+template <int END>
+__device__ __forceinline__ double2 fft_load(const Fft &f, uint32_t i) {
+    if constexpr (END == kEncFirst) {
+        const uint32_t j = f.iperm[i];
+        return j < f.n_values ? f.in[j] : double2{0.0, 0.0};
+    } else if constexpr (END == kDecFirst) {
+        const double2 v = f.in[i], z = f.zeta[i];  // z_k zeta^k
+        return double2{__builtin_fma(v.x, z.x, -(v.y * z.y)), __builtin_fma(v.x, z.y, v.y * z.x)};
+    } else {
+        return f.in[i];
+    }
+}
+
+template <int END>
+__device__ __forceinline__ void fft_store(const Fft &f, uint32_t i, double2 v, uint32_t &mb) {
+    if constexpr (END == kEncLast) {
+        const double2 z = f.zeta[i];  // w_k zeta^-k / M times the scale
+        const double s = -z.y;
+        const double re = __builtin_fma(v.x, z.x, -(v.y * s)) * f.scale;
+        const double im = __builtin_fma(v.x, s, v.y * z.x) * f.scale;
+        const uint32_t br = coeff_bits(re), bi = coeff_bits(im);
+        mb = max(mb, max(br, bi));
+        f.out[i] = double2{re, im};
+    } else if constexpr (END == kDecLast) {
+        f.out[f.iperm[i]] = v;
+    } else {
+        f.out[i] = v;
+    }
+}
+
+template <int S, int END>
+__global__ void __launch_bounds__(64) k_fft(Fft f) {
+    constexpr int PTS = 1 << S, COLS = 512 / PTS, RL = S % 3 ? S % 3 : 3, NR = (S - RL) / 3;  // NR rounds of 3, one of RL
+    constexpr bool FIRST = END == kEncFirst || END == kDecFirst;
+    __shared__ double2 lds[512 + 64];
+    const uint32_t col = threadIdx.x % COLS, tl = threadIdx.x / COLS;
+    const uint32_t c0 = blockIdx.x * COLS + col;
+    const uint32_t k0 = FIRST ? 0 : c0;
+    // point t of this column comes from c0 + t 2^(logm - S) in either half
+    const uint32_t step = f.logm - S;
+    auto at = [&](uint32_t i) { return (i + (i >> 3)) * COLS + col; };
+    if (END == kEncFirst && blockIdx.x == 0 && threadIdx.x == 0) *f.bits = 1;
+    double2 x[8];
+#pragma unroll
+    for (int u = 0; u < 8; u++) x[u] = fft_load<END>(f, c0 + ((tl + u * (PTS / 8)) << step));
+#pragma unroll
+    for (int r = 0; r < NR; r++) {
+        if (r) {
+#pragma unroll
+            for (int u = 0; u < 8; u++) x[u] = lds[at(tl + u * (PTS / 8))];
+            __syncthreads();
+        }
+        const uint32_t ls = 3 * r, k = tl & ((1u << ls) - 1);
+        fft_round<3>(x, k, ls, k0, f);
+#pragma unroll
+        for (int w = 0; w < 8; w++) lds[at(8 * (tl - k) + k + ((uint32_t)w << ls))] = x[w];
+        __syncthreads();
+    }
+    uint32_t mb = 1;
+    // the last round: 8 / 2^RL groups of 2^RL points, each at j + v PTS / 2^RL before and after
+#pragma unroll
+    for (int g = 0; g < (8 >> RL); g++) {
+        const uint32_t j = tl + g * (PTS / 8);
+        double2 z[1 << RL];
+#pragma unroll
+        for (int u = 0; u < (1 << RL); u++) z[u] = lds[at(j + u * (PTS >> RL))];
+        fft_round<RL>(z, j, S - RL, k0, f);
+#pragma unroll
+        for (int w = 0; w < (1 << RL); w++) {
+            const uint32_t p = j + w * (PTS >> RL);
+            fft_store<END>(f, FIRST ? c0 * PTS + p : c0 + (p << f.loga), z[w], mb);
+        }
+    }
+    if constexpr (END == kEncLast) {
+        for (int d = 32; d; d >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, d));
+        if (threadIdx.x == 0) atomicMax(f.bits, mb);
+    }
+}
+
+// The FFT's tables: exp(i pi t / (M / 2)), t < M / 2, then exp(i pi k / N), k < M.
+__global__ void k_fft_tables(double2 *tw, double2 *zeta, uint32_t M) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= M) return;
+    double s, c;
+    if (i < M / 2) {
+        sincospi((double)i / (double)(M / 2), &s, &c);
+        tw[i] = double2{c, s};
+    }
+    sincospi((double)i / (double)(2 * M), &s, &c);
+    zeta[i] = double2{c, s};
 }
 
 // a b mod q for any a, b < 2^64 (ratio = floor(2^128 / q))
@@ -87,58 +219,48 @@ __device__ __forceinline__ uint32_t coeff_bits(double v) {
     return (uint32_t)(m > 0.5 ? ex : ex - 1) + 1;
 }
 
-// z_k = w_k zeta^-k / M; coefficients -> RNS residues of the L first primes.
-// bits receives the largest coeff_bits of the unrounded coefficients.
-__global__ void k_enc_round(const double2 *w, uint64_t *out, const uint64_t *mod, const ulonglong2 *ratio,
-                            uint32_t L, uint32_t N, double scale_over_m, uint32_t *bits) {
-    const uint32_t M = N / 2;
-    uint32_t mb = 1;
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < M; k += gridDim.x * blockDim.x) {
-        double s, c;
-        sincospi(-(double)k / (double)N, &s, &c);  // zeta^-k = exp(-i pi k / N)
-        const double2 v = w[k];
-        const double re = (v.x * c - v.y * s) * scale_over_m;
-        const double im = (v.x * s + v.y * c) * scale_over_m;
-        const double u[2] = {re, im};
+// Unrounded coefficients u_k = (m_k, m_(k+M)) -> RNS residues of primes
+// [kLimbGroup blockIdx.y, ...) of the L first.  A thread a coefficient pair and
+// a few limbs: with all limbs in one thread, 2^14 pairs were 256 waves of a
+// chain of 2 L reductions each (12 limbs 14.9 -> 4.4 us).
+// Block (0, 0) hands the largest coeff_bits, complete here, to the host.
+constexpr uint32_t kLimbGroup = 2;
+__global__ void __launch_bounds__(kThreads)
+    k_enc_round(const double2 *u, uint64_t *out, const uint64_t *mod, const ulonglong2 *ratio, uint32_t L, uint32_t N,
+                const uint32_t *bits, uint32_t *host_bits) {
+    const uint32_t M = N / 2, k = blockIdx.x * kThreads + threadIdx.x;
+    if (k == 0 && blockIdx.y == 0) *host_bits = *bits;
+    const double2 v = u[k];
+    const double x[2] = {rint(v.x), rint(v.y)};
+    const uint32_t l0 = blockIdx.y * kLimbGroup, l1 = min(l0 + kLimbGroup, L);
+    for (uint32_t l = l0; l < l1; l++) {
+        const uint64_t q = mod[l];
+        const ulonglong2 rt = ratio[l];
         for (int h = 0; h < 2; h++) {
-            const uint32_t b = coeff_bits(u[h]);
-            mb = b > mb ? b : mb;
-            const double x = rint(u[h]);
-            const bool neg = x < 0;
-            const double a = b == ~0u ? 0.0 : fabs(x);
-            for (uint32_t l = 0; l < L; l++) {
-                const uint64_t q = mod[l];
-                uint64_t t = dbl_int_mod(a, q, ratio[l]);
-                if (neg && t) t = q - t;
-                out[(size_t)l * N + k + h * M] = t;
-            }
+            const double a = fabs(x[h]);
+            uint64_t t = dbl_int_mod(a < __builtin_huge_val() ? a : 0.0, q, rt);
+            if (x[h] < 0 && t) t = q - t;
+            out[(size_t)l * N + k + h * M] = t;
         }
     }
-    atomicMax(bits, mb);
 }
 
-// z_k = w_k zeta^-k / M -> the reference's level-independent single-chain
+// Unrounded coefficients -> the reference's level-independent single-chain
 // coefficients (src/single_chain_plaintext.cu:93-150): the rounded
 // coefficient's residue mod q0, centred into (-q0/2, q0/2].
-__global__ void k_enc_round_signed(const double2 *w, int64_t *out, uint32_t N, double scale_over_m, uint64_t q0,
-                                   ulonglong2 r0, uint32_t *bits) {
-    const uint32_t M = N / 2;
-    uint32_t mb = 1;
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < M; k += gridDim.x * blockDim.x) {
-        double s, c;
-        sincospi(-(double)k / (double)N, &s, &c);
-        const double2 v = w[k];
-        const double u[2] = {(v.x * c - v.y * s) * scale_over_m, (v.x * s + v.y * c) * scale_over_m};
-        for (int h = 0; h < 2; h++) {
-            const uint32_t b = coeff_bits(u[h]);
-            mb = b > mb ? b : mb;
-            const double x = rint(u[h]);
-            uint64_t t = dbl_int_mod(b == ~0u ? 0.0 : fabs(x), q0, r0);
-            if (x < 0 && t) t = q0 - t;
-            out[k + h * M] = t > q0 / 2 ? -(int64_t)(q0 - t) : (int64_t)t;
-        }
+__global__ void __launch_bounds__(kThreads)
+    k_enc_round_signed(const double2 *u, int64_t *out, uint32_t N, uint64_t q0, ulonglong2 r0, const uint32_t *bits,
+                       uint32_t *host_bits) {
+    const uint32_t M = N / 2, k = blockIdx.x * kThreads + threadIdx.x;
+    if (k == 0) *host_bits = *bits;
+    const double2 v = u[k];
+    const double x[2] = {rint(v.x), rint(v.y)};
+    for (int h = 0; h < 2; h++) {
+        const double a = fabs(x[h]);
+        uint64_t t = dbl_int_mod(a < __builtin_huge_val() ? a : 0.0, q0, r0);
+        if (x[h] < 0 && t) t = q0 - t;
+        out[k + h * M] = t > q0 / 2 ? -(int64_t)(q0 - t) : (int64_t)t;
     }
-    atomicMax(bits, mb);
 }
 
 // Coefficient i of the L coefficient-form limbs as a double times inv_scale,
@@ -187,43 +309,88 @@ __device__ double compose_one(uint64_t *coef, size_t i, const uint64_t *mod, con
     return neg ? -res : res;
 }
 
-// Coefficient-form limbs -> twisted complex vector w_k = z_k zeta^k, z_k = (m_k + i m_(k+M)) / scale.
-__global__ void k_dec_compose(uint64_t *coef, double2 *w, const uint64_t *mod, const ulonglong2 *ratio,
-                              const ulonglong2 *inv, uint32_t Q, uint32_t L, uint32_t N, double inv_scale) {
-    const uint32_t M = N / 2;
-    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < M; k += gridDim.x * blockDim.x) {
-        const double re = compose_one(coef, k, mod, ratio, inv, Q, L, N, inv_scale);
-        const double im = compose_one(coef, k + M, mod, ratio, inv, Q, L, N, inv_scale);
-        double s, c;
-        sincospi((double)k / (double)N, &s, &c);  // zeta^k
-        w[k] = double2{re * c - im * s, re * s + im * c};
+// Coefficient-form limbs -> z_k = (m_k + i m_(k+M)) / scale, a thread a coefficient.
+__global__ void __launch_bounds__(kThreads)
+    k_dec_compose(uint64_t *coef, double *z, const uint64_t *mod, const ulonglong2 *ratio, const ulonglong2 *inv,
+                  uint32_t Q, uint32_t L, uint32_t N, double inv_scale) {
+    const uint32_t M = N / 2, i = blockIdx.x * kThreads + threadIdx.x;
+    z[2 * (i & (M - 1)) + (i >= M)] = compose_one(coef, i, mod, ratio, inv, Q, L, N, inv_scale);
+}
+
+template <int END>
+void launch_fft(const Fft &f, uint32_t S, hipStream_t s) {
+    const dim3 grid((1u << f.logm) / 512), block(64);
+    switch (S) {
+        case 4: hipLaunchKernelGGL((k_fft<4, END>), grid, block, 0, s, f); break;
+        case 5: hipLaunchKernelGGL((k_fft<5, END>), grid, block, 0, s, f); break;
+        case 6: hipLaunchKernelGGL((k_fft<6, END>), grid, block, 0, s, f); break;
+        case 7: hipLaunchKernelGGL((k_fft<7, END>), grid, block, 0, s, f); break;
+        case 8: hipLaunchKernelGGL((k_fft<8, END>), grid, block, 0, s, f); break;
+        default: fail(PFA_ERR_INVALID_ARGUMENT, "unsupported FFT size");
     }
 }
 
-__global__ void k_zero_flag(uint32_t *p) { *p = 0; }
+// Both launches: `in` through `mid` to `out` (N is 2^10 .. 2^17, so either
+// part has 4 to 8 stages).
+template <int FIRST, int LAST>
+void fft(const Ctx &c, Fft f, const double2 *in, double2 *mid, double2 *out, hipStream_t s) {
+    f.tw = c.fft_tw;
+    f.zeta = c.fft_tw + c.N / 4;
+    f.iperm = c.slot_iperm;
+    f.logm = c.logN - 1;
+    const uint32_t s1 = f.logm / 2;
+    f.in = in;
+    f.out = mid;
+    f.loga = 0;
+    launch_fft<FIRST>(f, s1, s);
+    f.in = mid;
+    f.out = out;
+    f.loga = s1;
+    launch_fft<LAST>(f, f.logm - s1, s);
+}
 
-inline dim3 ew_grid(uint32_t n) { return dim3(std::min<uint32_t>((n + kThreads - 1) / kThreads, 4096)); }
+// Slots -> unrounded coefficients (m_k, m_(k+M)) in w, the largest coeff_bits in *bits.
+double2 *encode_coeffs_f64(const Ctx &c, Scratch &sc, const double *values, size_t n_values, double scale,
+                           uint32_t *bits, hipStream_t s) {
+    const uint32_t M = c.N / 2;
+    double2 *buf = sc.alloc<double2>(2 * (size_t)M);
+    Fft f{};
+    f.sign = -1.0;
+    f.n_values = (uint32_t)n_values;
+    f.scale = scale / (double)M;
+    f.bits = bits;
+    fft<kEncFirst, kEncLast>(c, f, (const double2 *)values, buf, buf + M, s);
+    return buf + M;
+}
 
-// In-place (ping-pong) length-M FFT; returns the buffer holding the result.
-double2 *fft(double2 *a, double2 *b, uint32_t M, double sign, hipStream_t s) {
-    for (uint32_t Ns = 1; Ns < M; Ns <<= 1) {
-        hipLaunchKernelGGL(k_fft_stage, ew_grid(M / 2), dim3(kThreads), 0, s, a, b, M, Ns, sign);
-        std::swap(a, b);
+// The arena's mapped host word, which a kernel of stream s writes and the host
+// reads after waiting for s: a copy from device memory waits for its own
+// launch as well.
+uint32_t *host_word(Arena &a, uint32_t **dev) {
+    if (!a.word) {
+        PFA_HIP(hipHostMalloc((void **)&a.word, 64, hipHostMallocMapped));
+        PFA_HIP(hipHostGetDevicePointer((void **)&a.word_dev, a.word, 0));
     }
-    return a;
+    *dev = a.word_dev;
+    return a.word;
 }
 
 }  // namespace
 
 void encoder_init(Ctx &c) {
     const uint32_t M = c.N / 2, m2 = 2 * c.N;
-    std::vector<uint32_t> perm(M);
+    std::vector<uint32_t> iperm(M);
     uint64_t p = 1;
     for (uint32_t j = 0; j < M; j++) {
-        perm[j] = (uint32_t)((p - 1) / 4);
+        iperm[(p - 1) / 4] = j;
         p = (p * 5) % m2;
     }
-    c.slot_perm = c.upload(perm);
+    c.slot_iperm = c.upload(iperm);
+    c.fft_tw = c.upload(std::vector<double2>(M / 2 + M));
+    hipLaunchKernelGGL(k_fft_tables, dim3((M + kThreads - 1) / kThreads), dim3(kThreads), 0, hipStreamPerThread,
+                       c.fft_tw, c.fft_tw + M / 2, M);
+    PFA_HIP(hipGetLastError());
+    PFA_HIP(hipStreamSynchronize(hipStreamPerThread));
     std::vector<ulonglong2> inv((size_t)c.Q * c.Q, ulonglong2{0, 0});
     for (uint32_t i = 0; i < c.Q; i++)
         for (uint32_t j = i + 1; j < c.Q; j++) {
@@ -275,21 +442,16 @@ int pfa_ckks_encode(const pfa_context *ctx, const double *values, size_t n_value
         check_scale(scale, tb, 1);
         const hipStream_t s = as_stream(stream);
         Scratch sc(c, s);
-        double2 *buf = sc.alloc<double2>(2 * (size_t)M);
-        uint32_t *flag = sc.alloc<uint32_t>(1);
-        hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(1), 0, s, flag);
-        hipLaunchKernelGGL(k_enc_scatter, ew_grid(M), dim3(kThreads), 0, s, (const double2 *)values,
-                           (uint32_t)n_values, buf, c.slot_perm, M);
-        double2 *w = fft(buf, buf + M, M, -1.0, s);
-        hipLaunchKernelGGL(k_enc_round, ew_grid(M), dim3(kThreads), 0, s, w, out, c.mod, c.ratio, (uint32_t)L, c.N,
-                           scale / (double)M, flag);
+        uint32_t *flag = sc.alloc<uint32_t>(1), *word_dev;
+        const volatile uint32_t *word = host_word(arena_for(c, s), &word_dev);
+        const double2 *u = encode_coeffs_f64(c, sc, values, n_values, scale, flag, s);
+        hipLaunchKernelGGL(k_enc_round, dim3(M / kThreads, ((uint32_t)L + kLimbGroup - 1) / kLimbGroup),
+                           dim3(kThreads), 0, s, u, out, c.mod, c.ratio, (uint32_t)L, c.N, flag, word_dev);
         PFA_HIP(hipGetLastError());
-        uint32_t h_flag = 0;
-        PFA_HIP(hipMemcpyAsync(&h_flag, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        PFA_HIP(hipStreamSynchronize(s));
-        require(h_flag < tb, "encoded values are too large");  // src/ckks.cu:122-126
         NttLaunch fw{out, out, 0, 0, 1, (uint32_t)L};
         ntt_forward(c, fw, s);
+        PFA_HIP(hipStreamSynchronize(s));
+        require(*word < tb, "encoded values are too large");  // src/ckks.cu:122-126
     });
 }
 
@@ -306,19 +468,14 @@ int pfa_ckks_encode_coeffs(const pfa_context *ctx, const double *values, size_t 
         check_scale(scale, tb, 1);
         const hipStream_t s = as_stream(stream);
         Scratch sc(c, s);
-        double2 *buf = sc.alloc<double2>(2 * (size_t)M);
-        uint32_t *flag = sc.alloc<uint32_t>(1);
-        hipLaunchKernelGGL(k_zero_flag, dim3(1), dim3(1), 0, s, flag);
-        hipLaunchKernelGGL(k_enc_scatter, ew_grid(M), dim3(kThreads), 0, s, (const double2 *)values,
-                           (uint32_t)n_values, buf, c.slot_perm, M);
-        double2 *w = fft(buf, buf + M, M, -1.0, s);
-        hipLaunchKernelGGL(k_enc_round_signed, ew_grid(M), dim3(kThreads), 0, s, w, coeffs, c.N, scale / (double)M,
-                           c.moduli[0], host_ratio(c.moduli[0]), flag);
+        uint32_t *flag = sc.alloc<uint32_t>(1), *word_dev;
+        const volatile uint32_t *word = host_word(arena_for(c, s), &word_dev);
+        const double2 *u = encode_coeffs_f64(c, sc, values, n_values, scale, flag, s);
+        hipLaunchKernelGGL(k_enc_round_signed, dim3(M / kThreads), dim3(kThreads), 0, s, u, coeffs, c.N, c.moduli[0],
+                           host_ratio(c.moduli[0]), flag, word_dev);
         PFA_HIP(hipGetLastError());
-        uint32_t h_flag = 0;
-        PFA_HIP(hipMemcpyAsync(&h_flag, flag, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
         PFA_HIP(hipStreamSynchronize(s));
-        require(h_flag < tb, "encoded values are too large");
+        require(*word < tb, "encoded values are too large");
     });
 }
 
@@ -335,10 +492,11 @@ int pfa_ckks_decode(const pfa_context *ctx, const uint64_t *in, size_t L, double
         double2 *buf = sc.alloc<double2>(2 * (size_t)M);
         NttLaunch inv{in, coef, 0, 0, 1, (uint32_t)L};
         ntt_inverse(c, inv, s);
-        hipLaunchKernelGGL(k_dec_compose, ew_grid(M), dim3(kThreads), 0, s, coef, buf, c.mod, c.ratio, c.crt_inv, c.Q,
-                           (uint32_t)L, c.N, 1.0 / scale);
-        double2 *W = fft(buf, buf + M, M, 1.0, s);
-        hipLaunchKernelGGL(k_dec_gather, ew_grid(M), dim3(kThreads), 0, s, W, (double2 *)values, c.slot_perm, M);
+        hipLaunchKernelGGL(k_dec_compose, dim3(c.N / kThreads), dim3(kThreads), 0, s, coef, (double *)buf, c.mod, c.ratio,
+                           c.crt_inv, c.Q, (uint32_t)L, c.N, 1.0 / scale);
+        Fft f{};
+        f.sign = 1.0;
+        fft<kDecFirst, kDecLast>(c, f, buf, buf + M, (double2 *)values, s);
         PFA_HIP(hipGetLastError());
     });
 }

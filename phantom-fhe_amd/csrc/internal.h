@@ -138,6 +138,8 @@ struct Arena {
     // arrival counters of the inner product's split items (k_inner_ws), zero
     // between launches (the last arrival clears its counter)
     uint32_t *ws_counter = nullptr;
+    // mapped pinned host word of the encoder's size check, allocated on first use
+    uint32_t *word = nullptr, *word_dev = nullptr;
 };
 
 struct Ctx {
@@ -198,7 +200,8 @@ struct Ctx {
     ulonglong2 *mdr_bc = nullptr;
     // key construction: [P]_{q_i} Shoup pairs over all QP rows (0 on P rows)
     ulonglong2 *pmodq = nullptr;
-    uint32_t *slot_perm = nullptr;   // [N/2] CKKS slot j -> DFT index (5^j mod 2N - 1) / 4
+    uint32_t *slot_iperm = nullptr;  // [N/2] DFT index (5^j mod 2N - 1) / 4 -> CKKS slot j
+    double2 *fft_tw = nullptr;       // [N/4] exp(4 pi i t / N), then [N/2] exp(pi i k / N)
     ulonglong2 *crt_inv = nullptr;   // [Q][Q] q_i^-1 mod q_j (i < j) as Shoup pairs: the decoder's Garner composition
     std::vector<Level> levels;  // index = chain index (0 unused)
     std::vector<void *> allocations;
