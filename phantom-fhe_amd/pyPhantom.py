@@ -792,9 +792,8 @@ class ckks_encoder:
     def slot_count(self) -> int:
         return self._slots
 
-    def _encode(self, ctx, values, scale, chain_index):
+    def _encode(self, ctx, v, scale, chain_index):
         t = _torch()
-        v = np.asarray(values, dtype=np.complex128).ravel()
         if v.size == 0:
             raise ValueError("Input vector is empty")
         if v.size > self._slots:
@@ -803,29 +802,29 @@ class ckks_encoder:
             raise ValueError("chain index out of range")
         L = ctx.size_Ql(chain_index)
         out = ctx._empty(L, ctx.N)
-        ctx.native.ckks_encode(t.from_numpy(v).to(ctx.dev), scale, out, L)
+        ctx.native.ckks_encode(t.from_numpy(v).to(ctx.dev).to(t.complex128), scale, out, L)
         pt = plaintext()
         pt.data, pt._chain_index, pt._scale = out, chain_index, float(scale)
         return pt
 
     def encode_double_vector(self, ctx, values, scale, chain_index=1):
-        return self._encode(ctx, np.asarray(values, dtype=np.float64), scale, chain_index)
+        # a copy (from_numpy takes neither read-only nor reversed memory); real values widen on the device
+        return self._encode(ctx, np.array(values, dtype=np.float64, order="C").ravel(), scale, chain_index)
 
     def encode_complex_vector(self, ctx, values, scale, chain_index=1):
-        return self._encode(ctx, values, scale, chain_index)
+        return self._encode(ctx, np.asarray(values, dtype=np.complex128).ravel(), scale, chain_index)
 
     def _decode(self, ctx, pt):
         t = _torch()
         out = t.empty(self._slots, dtype=t.complex128, device=ctx.dev)
         ctx.native.ckks_decode(pt.data, pt.data.shape[0], pt.scale(), out)
-        t.cuda.synchronize(ctx.dev)
-        return out.cpu().numpy()
+        return out
 
     def decode_complex_vector(self, ctx, pt):
-        return self._decode(ctx, pt).tolist()
+        return self._decode(ctx, pt).cpu().numpy().tolist()
 
     def decode_double_vector(self, ctx, pt):
-        return self._decode(ctx, pt).real.tolist()
+        return self._decode(ctx, pt).real.contiguous().cpu().numpy().tolist()
 
 
 # ---------------------------------------------------------------- evaluator

@@ -81,3 +81,29 @@ def test_encode_refuses_what_does_not_fit():
             enc.encode_double_vector(ctx, v * bad, 2.0 ** 40, 1)
         pt = enc.encode_double_vector(ctx, v, 2.0 ** 40, 1)
         assert np.abs(np.array(enc.decode_double_vector(ctx, pt)) - 1).max() < 1e-9
+
+
+@pytest.mark.parametrize("form", ["list", "reversed", "readonly", "strided", "float32", "2d"])
+def test_real_vectors_as_complex_ones(form):
+    """encode_double_vector gives encode_complex_vector's plaintext for any array or list of reals, and
+    decode_double_vector the real parts of decode_complex_vector."""
+    import pyPhantom as ph
+    import torch
+
+    n = 1 << 11
+    p = ph.params(ph.scheme_type.ckks)
+    p.set_poly_modulus_degree(n)
+    p.set_coeff_modulus(ph.create_coeff_modulus(n, [60, 40, 50, 60]))
+    p.set_special_modulus_size(1)
+    ctx = ph.context(p)
+    enc = ph.ckks_encoder(ctx)
+    v = np.random.default_rng(5).uniform(-1, 1, 600)
+    if form == "readonly":
+        v.flags.writeable = False
+    x = {"list": v.tolist(), "reversed": v[::-1], "readonly": v, "strided": v[::3], "float32": v.astype(np.float32),
+         "2d": v.reshape(20, 30).T}[form]
+    a = enc.encode_double_vector(ctx, x, 2.0 ** 40)
+    b = enc.encode_complex_vector(ctx, np.array(x, dtype=np.complex128), 2.0 ** 40)
+    assert torch.equal(a.data.view(torch.int64), b.data.view(torch.int64))
+    got = enc.decode_double_vector(ctx, a)
+    assert isinstance(got, list) and got == [z.real for z in enc.decode_complex_vector(ctx, b)]
