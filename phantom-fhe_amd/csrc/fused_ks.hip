@@ -1212,7 +1212,7 @@ __device__ __forceinline__ void tensor_rows_tile(const TensorRows &a, RowStage<S
         }
     }
     __syncthreads();
-    const StagedTw w = RS::view(twl, a.itw, threadIdx.x / Sub<S2>::T);
+    const auto w = RS::view(twl, a.itw, threadIdx.x / Sub<S2>::T);
     inv_rows_lds<A, S1, S2, R, true, R>(w, r, q, lds, a.mid + r.m * a.mid_stride + (size_t)r.l * G::N,
                                         threadIdx.x < NR);
 }
@@ -1547,7 +1547,7 @@ k_galois_rows(GaloisRows a, NttTables t) {
     // the staged twiddles were requested first: this waits for them only
     stage.st.store(twl);
     uint64_t *mid = a.mid + ((size_t)i * a.Ql + r.l) * G::N;
-    const StagedTw w = RS::view(twl, t.itw + (size_t)r.l * G::N, threadIdx.x / Sub<S2>::T);
+    const auto w = RS::view(twl, t.itw + (size_t)r.l * G::N, threadIdx.x / Sub<S2>::T);
     if (q < kF64PrimeBound) {
         const ArithF64 ar(q);
 #pragma unroll

@@ -24,6 +24,8 @@
 // the limb's twiddles.
 #pragma once
 
+#include <type_traits>
+
 #include "modarith.h"
 
 namespace pfa {
@@ -148,20 +150,52 @@ __device__ __forceinline__ void inv_guard(typename A::T (&x)[E], const A &ar) {
     }
 }
 
-// forward, stages g = 0 .. LE-1 on elements u = F + T e
+template <class A, int S>
+__device__ __forceinline__ void fwd_stage_a(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
+                                            uint32_t base, int g) {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+    const int d = E >> (g + 1);
+    fwd_guard(x, ar, g);
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        if (e & d) continue;
+        ar.ct(x[e], x[e + d], tw[(base << g) + (e >> (LE - g))]);
+    }
+}
+
+template <class A, int S>
+__device__ __forceinline__ void fwd_stage_b(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
+                                            uint32_t base, uint32_t F, int g) {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+    const int d = 1 << (S - 1 - g);
+    const ulonglong2 *t = tw + (base << g) + (F << (LE - S + g));
+    fwd_guard(x, ar, g - LE);
+#pragma unroll
+    for (int e = 0; e < E; e++) {
+        if (e & d) continue;
+        ar.ct(x[e], x[e + d], t[e >> (S - g)]);
+    }
+}
+
+// forward, stages g = 0 .. LE-1 on elements u = F + T e.  The stages of 32
+// elements (N = 2^17) are written out, here and in fwd_round_b: as a loop they
+// pass the compiler's unrolling limit in the integer policy, and the elements,
+// indexed at run time, live in scratch memory (272 bytes a lane; 35 limbs of
+// 55-bit primes forward 159 us, written out 55.5 us).
 template <class A, int S>
 __device__ __forceinline__ void fwd_round_a(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
                                             uint32_t base) {
-    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+    constexpr int LE = Sub<S>::LE;
+    static_assert(LE <= 5, "write the sixth stage out");
+    if constexpr (LE == 5) {
+        fwd_stage_a<A, S>(x, ar, tw, base, 0);
+        fwd_stage_a<A, S>(x, ar, tw, base, 1);
+        fwd_stage_a<A, S>(x, ar, tw, base, 2);
+        fwd_stage_a<A, S>(x, ar, tw, base, 3);
+        fwd_stage_a<A, S>(x, ar, tw, base, 4);
+    } else {
 #pragma unroll
-    for (int g = 0; g < LE; g++) {
-        const int d = E >> (g + 1);
-        fwd_guard(x, ar, g);
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            if (e & d) continue;
-            ar.ct(x[e], x[e + d], tw[(base << g) + (e >> (LE - g))]);
-        }
+        for (int g = 0; g < LE; g++) fwd_stage_a<A, S>(x, ar, tw, base, g);
     }
 }
 
@@ -169,17 +203,16 @@ __device__ __forceinline__ void fwd_round_a(typename A::T (&x)[Sub<S>::E], const
 template <class A, int S>
 __device__ __forceinline__ void fwd_round_b(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
                                             uint32_t base, uint32_t F) {
-    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+    constexpr int LE = Sub<S>::LE;
+    if constexpr (LE == 5) {
+        static_assert(S == 9, "stages 5 to 8");
+        fwd_stage_b<A, S>(x, ar, tw, base, F, 5);
+        fwd_stage_b<A, S>(x, ar, tw, base, F, 6);
+        fwd_stage_b<A, S>(x, ar, tw, base, F, 7);
+        fwd_stage_b<A, S>(x, ar, tw, base, F, 8);
+    } else {
 #pragma unroll
-    for (int g = LE; g < S; g++) {
-        const int d = 1 << (S - 1 - g);
-        const ulonglong2 *t = tw + (base << g) + (F << (LE - S + g));
-        fwd_guard(x, ar, g - LE);
-#pragma unroll
-        for (int e = 0; e < E; e++) {
-            if (e & d) continue;
-            ar.ct(x[e], x[e + d], t[e >> (S - g)]);
-        }
+        for (int g = LE; g < S; g++) fwd_stage_b<A, S>(x, ar, tw, base, F, g);
     }
 }
 
@@ -270,10 +303,12 @@ struct TableTwB {
     }
 };
 
-// The integer rounds with their twiddles in W (LdsTwA, TwB, TableTwB)
+// The integer rounds with their twiddles in W (LdsTwA, TwB, TableTwB), for up
+// to 16 elements a thread (as loops over the stages: see fwd_round_a)
 template <int S, class W>
 __device__ __forceinline__ void fwd_round_a_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const W &w) {
     constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+    static_assert(LE <= 4);
 #pragma unroll
     for (int g = 0; g < LE; g++) {
         const int d = E >> (g + 1);
@@ -291,6 +326,7 @@ __device__ __forceinline__ void fwd_round_a_int(uint64_t (&x)[Sub<S>::E], const 
 template <int S, class W>
 __device__ __forceinline__ void fwd_round_b_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const W &w) {
     constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
+    static_assert(LE <= 4);
 #pragma unroll
     for (int g = LE; g < S; g++) {
         const int d = 1 << (S - 1 - g);
@@ -598,17 +634,19 @@ struct TwStage {
 };
 
 // Staged entries of a rows-pass tile.  FP64 policy: rb[g][tile R + i] for
-// g < S2, i < R, then the small table's first 2^(S2-1) entries; integer policy:
-// the first-round entries (LdsTwA) of the R rows, E slots a row.
-template <int S1, int S2, int R = Geo<S1, S2>::ROWS>
+// g < S2, i < R, then the small table's first 2^(S2-1) entries; integer policy
+// with INT: the first-round entries (LdsTwA) of the R rows, E slots a row (not
+// for 32 elements a thread, N = 2^17, whose rounds read the full table).
+template <int S1, int S2, int R = Geo<S1, S2>::ROWS, bool INT = (Sub<S2>::LE <= 4)>
 struct RowStage {
     using G = Geo<S1, S2>;
+    using View = std::conditional_t<INT, StagedTw, TileTw>;
     static constexpr int RB = S2 * R, E = Sub<S2>::E;
-    static constexpr int NF = RB + (1 << (S2 - 1)), NI = R * E;
+    static constexpr int NF = RB + (1 << (S2 - 1)), NI = INT ? R * E : 0;
     static constexpr int N = NF > NI ? NF : NI;
     TwStage<N, R * Sub<S2>::T> st;
     __device__ __forceinline__ void load(const NttTables &t, uint32_t prow, uint32_t tile, bool fwd, uint64_t q) {
-        if (q < kF64PrimeBound) {
+        if (!INT || q < kF64PrimeBound) {
             const ulonglong2 *rb = (fwd ? t.rb_fw : t.rb_inv) + (size_t)prow * S2 * G::N1 + tile * R;
             const ulonglong2 *small = (fwd ? t.small_fw : t.small_inv) + (size_t)prow * kSmall;
             st.load([&](uint32_t i) {
@@ -625,8 +663,12 @@ struct RowStage {
     }
     // LDS copy -> the tile's twiddle view (full: the prime's global table, for
     // the integer policy's second round)
-    __device__ __forceinline__ static StagedTw view(const ulonglong2 *lds, const ulonglong2 *full, uint32_t rr) {
-        return StagedTw{{nullptr, full, lds, lds + RB, rr}, lds + rr * E};
+    __device__ __forceinline__ static View view(const ulonglong2 *lds, const ulonglong2 *full, uint32_t rr) {
+        const TileTw w{nullptr, full, lds, lds + RB, rr};
+        if constexpr (INT)
+            return StagedTw{w, lds + rr * E};
+        else
+            return w;
     }
 };
 
@@ -831,7 +873,7 @@ ntt_fwd_rows(NttBatch b, NttTables t) {
         for (int e = 0; e < SB::E; e++) raw[e] = ld_stream(&s[F + SB::T * e]);
         stage.st.store(twl);
         __syncthreads();
-        const StagedTw w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
+        const auto w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
         uint64_t *olimb = b.dst + r.m * b.dstride + (size_t)r.l * G::N;
         if (q < kF64PrimeBound)
             fwd_rows_tile<ArithF64, S1, S2, R, R>(raw, w, r, q, lds, olimb);
@@ -861,7 +903,7 @@ __device__ __forceinline__ void inv_rows_lds(const TW &w, const TileRef &r, uint
     T x[SB::E];
     // integer twiddles: the second round's (this one's first) requested
     // together, the first round's from LDS
-    constexpr bool PRE = !A::kF64 && TW::kStaged && SB::LE <= 4;
+    constexpr bool PRE = !A::kF64 && TW::kStaged;
     if (active) {
 #pragma unroll
         for (int e = 0; e < SB::E; e++) x[e] = lr[rpad(F * SB::E + e)];
@@ -982,7 +1024,7 @@ ntt_inv_rows_staged(NttBatch b, NttTables t) {
         for (int e = 0; e < SB::E; e++) raw[e] = ld_stream(&s[F + SB::T * e]);
         stage.st.store(twl);
         __syncthreads();
-        const StagedTw w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
+        const auto w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
         uint64_t *olimb = b.dst + r.m * b.dstride + (size_t)r.l * G::N;
         if (q < kF64PrimeBound)
             inv_rows_tile<ArithF64, S1, S2, R, true, R>(raw, w, r, q, lds, olimb);
@@ -1272,7 +1314,7 @@ struct FlowJob {
             for (int e = 0; e < S2B::E; e++) raw[e] = ld_stream(&s[F + S2B::T * e]);
             stage.st.store(twl);
             __syncthreads();
-            const StagedTw w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
+            const auto w = RS::view(twl, t.itw + (size_t)prow * G::N, rr);
             if (q < kF64PrimeBound)
                 inv_rows_tile<ArithF64, S1, S2, G::ROWS, false>(raw, w, r, q, lds, limb);
             else
@@ -1295,7 +1337,7 @@ struct FlowJob {
             for (int e = 0; e < S2B::E; e++) raw[e] = s[F + S2B::T * e];
             stage.st.store(twl);
             __syncthreads();
-            const StagedTw w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
+            const auto w = RS::view(twl, t.tw + (size_t)prow * G::N, rr);
             if (q < kF64PrimeBound)
                 fwd_rows_tile<ArithF64, S1, S2, G::ROWS>(raw, w, r, q, lds, limb);
             else

@@ -1,0 +1,54 @@
+"""What the compiler made of the kernels, read from the built library's own gfx950 code objects: registers and
+scratch memory.  A thread's elements live in registers only while every loop over them unrolls; one that does not
+indexes them at run time, and they silently move to scratch memory with the same results at a fraction of the
+speed."""
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+LLVM = "/opt/rocm/llvm/bin"
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{kernel name with template arguments: {".vgpr_count": ..., ...}} of every code object in the library."""
+    import pfa_native as P
+
+    P.lib()
+    blob = open(P.LIB_PATH, "rb").read()
+    out = {}
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    at = blob.find(magic)
+    while at >= 0:
+        (count,) = struct.unpack_from("<Q", blob, at + len(magic))
+        entry = at + len(magic) + 8
+        for _ in range(count):
+            offset, size, length = struct.unpack_from("<QQQ", blob, entry)
+            triple = blob[entry + 24:entry + 24 + length].decode()
+            entry += 24 + length
+            if "gfx950" in triple and size:
+                path = tmp_path_factory.mktemp("code") / "object"
+                path.write_bytes(blob[at + offset:at + offset + size])
+                notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", str(path)], check=True,
+                                       capture_output=True, text=True).stdout
+                for block in re.split(r"\n  - (?=\.)", notes)[1:]:
+                    fields = dict(re.findall(r"^ {0,4}(\.\w+): +(\S+)$", block, re.M))
+                    if ".private_segment_fixed_size" in fields:
+                        out[fields[".name"]] = fields
+        at = blob.find(magic, at + 1)
+    names = subprocess.run(["c++filt"], input="\n".join(out), check=True,
+                           capture_output=True, text=True).stdout.split("\n")
+    plain = [re.sub(r"pfa::|\(anonymous namespace\)::|^void ", "", n).split("(")[0] for n in names]
+    out = {p: f for p, f in zip(plain, out.values())}
+    assert len(out) > 100
+    return out
+
+
+@pytest.mark.parametrize("kernel", ["ntt_fwd_rows<8, 9, 8>", "ntt_inv_rows<8, 9, 8>", "ntt_inv_rows_staged<8, 9, 8>",
+                                    "ntt_fwd_cols<8, 9>", "ntt_inv_cols<8, 9>", "k_epi_rows<8, 9>"])
+def test_largest_ring_elements_in_registers(kernels, kernel):
+    """N = 2^17: 32 elements a thread, the longest unrolled rounds."""
+    assert int(kernels[kernel][".private_segment_fixed_size"]) == 0
