@@ -150,52 +150,20 @@ __device__ __forceinline__ void inv_guard(typename A::T (&x)[E], const A &ar) {
     }
 }
 
-template <class A, int S>
-__device__ __forceinline__ void fwd_stage_a(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
-                                            uint32_t base, int g) {
-    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
-    const int d = E >> (g + 1);
-    fwd_guard(x, ar, g);
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        if (e & d) continue;
-        ar.ct(x[e], x[e + d], tw[(base << g) + (e >> (LE - g))]);
-    }
-}
-
-template <class A, int S>
-__device__ __forceinline__ void fwd_stage_b(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
-                                            uint32_t base, uint32_t F, int g) {
-    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
-    const int d = 1 << (S - 1 - g);
-    const ulonglong2 *t = tw + (base << g) + (F << (LE - S + g));
-    fwd_guard(x, ar, g - LE);
-#pragma unroll
-    for (int e = 0; e < E; e++) {
-        if (e & d) continue;
-        ar.ct(x[e], x[e + d], t[e >> (S - g)]);
-    }
-}
-
-// forward, stages g = 0 .. LE-1 on elements u = F + T e.  The stages of 32
-// elements (N = 2^17) are written out, here and in fwd_round_b: as a loop they
-// pass the compiler's unrolling limit in the integer policy, and the elements,
-// indexed at run time, live in scratch memory (272 bytes a lane; 35 limbs of
-// 55-bit primes forward 159 us, written out 55.5 us).
+// forward, stages g = 0 .. LE-1 on elements u = F + T e
 template <class A, int S>
 __device__ __forceinline__ void fwd_round_a(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
                                             uint32_t base) {
-    constexpr int LE = Sub<S>::LE;
-    static_assert(LE <= 5, "write the sixth stage out");
-    if constexpr (LE == 5) {
-        fwd_stage_a<A, S>(x, ar, tw, base, 0);
-        fwd_stage_a<A, S>(x, ar, tw, base, 1);
-        fwd_stage_a<A, S>(x, ar, tw, base, 2);
-        fwd_stage_a<A, S>(x, ar, tw, base, 3);
-        fwd_stage_a<A, S>(x, ar, tw, base, 4);
-    } else {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
 #pragma unroll
-        for (int g = 0; g < LE; g++) fwd_stage_a<A, S>(x, ar, tw, base, g);
+    for (int g = 0; g < LE; g++) {
+        const int d = E >> (g + 1);
+        fwd_guard(x, ar, g);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            if (e & d) continue;
+            ar.ct(x[e], x[e + d], tw[(base << g) + (e >> (LE - g))]);
+        }
     }
 }
 
@@ -203,16 +171,17 @@ __device__ __forceinline__ void fwd_round_a(typename A::T (&x)[Sub<S>::E], const
 template <class A, int S>
 __device__ __forceinline__ void fwd_round_b(typename A::T (&x)[Sub<S>::E], const A &ar, const ulonglong2 *tw,
                                             uint32_t base, uint32_t F) {
-    constexpr int LE = Sub<S>::LE;
-    if constexpr (LE == 5) {
-        static_assert(S == 9, "stages 5 to 8");
-        fwd_stage_b<A, S>(x, ar, tw, base, F, 5);
-        fwd_stage_b<A, S>(x, ar, tw, base, F, 6);
-        fwd_stage_b<A, S>(x, ar, tw, base, F, 7);
-        fwd_stage_b<A, S>(x, ar, tw, base, F, 8);
-    } else {
+    constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
 #pragma unroll
-        for (int g = LE; g < S; g++) fwd_stage_b<A, S>(x, ar, tw, base, F, g);
+    for (int g = LE; g < S; g++) {
+        const int d = 1 << (S - 1 - g);
+        const ulonglong2 *t = tw + (base << g) + (F << (LE - S + g));
+        fwd_guard(x, ar, g - LE);
+#pragma unroll
+        for (int e = 0; e < E; e++) {
+            if (e & d) continue;
+            ar.ct(x[e], x[e + d], t[e >> (S - g)]);
+        }
     }
 }
 
@@ -303,12 +272,10 @@ struct TableTwB {
     }
 };
 
-// The integer rounds with their twiddles in W (LdsTwA, TwB, TableTwB), for up
-// to 16 elements a thread (as loops over the stages: see fwd_round_a)
+// The integer rounds with their twiddles in W (LdsTwA, TwB, TableTwB)
 template <int S, class W>
 __device__ __forceinline__ void fwd_round_a_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const W &w) {
     constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
-    static_assert(LE <= 4);
 #pragma unroll
     for (int g = 0; g < LE; g++) {
         const int d = E >> (g + 1);
@@ -326,7 +293,6 @@ __device__ __forceinline__ void fwd_round_a_int(uint64_t (&x)[Sub<S>::E], const 
 template <int S, class W>
 __device__ __forceinline__ void fwd_round_b_int(uint64_t (&x)[Sub<S>::E], const ArithInt &ar, const W &w) {
     constexpr int LE = Sub<S>::LE, E = Sub<S>::E;
-    static_assert(LE <= 4);
 #pragma unroll
     for (int g = LE; g < S; g++) {
         const int d = 1 << (S - 1 - g);
@@ -635,8 +601,11 @@ struct TwStage {
 
 // Staged entries of a rows-pass tile.  FP64 policy: rb[g][tile R + i] for
 // g < S2, i < R, then the small table's first 2^(S2-1) entries; integer policy
-// with INT: the first-round entries (LdsTwA) of the R rows, E slots a row (not
-// for 32 elements a thread, N = 2^17, whose rounds read the full table).
+// with INT: the first-round entries (LdsTwA) of the R rows, E slots a row.  With
+// INT the entries a tile needs are known only with its prime, which FP64 tiles
+// then wait for too; at N = 2^17 (32 elements a thread) the integer policy reads
+// the table instead (forward, 35 limbs, staged / table: 50-bit primes 40.3 /
+// 39.8 us, 55-bit ones 50.7 / 56.0 us).
 template <int S1, int S2, int R = Geo<S1, S2>::ROWS, bool INT = (Sub<S2>::LE <= 4)>
 struct RowStage {
     using G = Geo<S1, S2>;

@@ -1,7 +1,6 @@
 """What the compiler made of the kernels, read from the built library's own gfx950 code objects: registers and
-scratch memory.  A thread's elements live in registers only while every loop over them unrolls; one that does not
-indexes them at run time, and they silently move to scratch memory with the same results at a fraction of the
-speed."""
+scratch memory.  A thread's elements live in registers only while every loop over them unrolls in time; one that
+does not leaves them in scratch memory, silently, with the same results at a fraction of the speed."""
 import os
 import re
 import struct
@@ -48,7 +47,8 @@ def kernels(tmp_path_factory):
 
 
 @pytest.mark.parametrize("kernel", ["ntt_fwd_rows<8, 9, 8>", "ntt_inv_rows<8, 9, 8>", "ntt_inv_rows_staged<8, 9, 8>",
-                                    "ntt_fwd_cols<8, 9>", "ntt_inv_cols<8, 9>", "k_epi_rows<8, 9>"])
+                                    "ntt_fwd_cols<8, 9>", "ntt_inv_cols<8, 9>", "k_epi_rows<8, 9>",
+                                    "k_inner_ws<8, 9>"])
 def test_largest_ring_elements_in_registers(kernels, kernel):
-    """N = 2^17: 32 elements a thread, the longest unrolled rounds."""
+    """N = 2^17: 32 elements a thread (64 sums in the inner product), the longest unrolled loops."""
     assert int(kernels[kernel][".private_segment_fixed_size"]) == 0
