@@ -13,7 +13,8 @@ LLVM = "/opt/rocm/llvm/bin"
 
 @pytest.fixture(scope="module")
 def kernels(tmp_path_factory):
-    """{kernel name with template arguments: {".vgpr_count": ..., ...}} of every code object in the library."""
+    """{kernel name with template arguments: {".vgpr_count": ..., ...}} of every code object in the library, with the
+    path of that code object as "object"."""
     import pfa_native as P
 
     P.lib()
@@ -36,7 +37,7 @@ def kernels(tmp_path_factory):
                 for block in re.split(r"\n  - (?=\.)", notes)[1:]:
                     fields = dict(re.findall(r"^ {0,4}(\.\w+): +(\S+)$", block, re.M))
                     if ".private_segment_fixed_size" in fields:
-                        out[fields[".name"]] = fields
+                        out[fields[".name"]] = {**fields, "object": str(path)}
         at = blob.find(magic, at + 1)
     names = subprocess.run(["c++filt"], input="\n".join(out), check=True,
                            capture_output=True, text=True).stdout.split("\n")
@@ -52,3 +53,24 @@ def kernels(tmp_path_factory):
 def test_largest_ring_elements_in_registers(kernels, kernel):
     """N = 2^17: 32 elements a thread (64 sums in the inner product), the longest unrolled loops."""
     assert int(kernels[kernel][".private_segment_fixed_size"]) == 0
+
+
+def _instructions(kernel):
+    text = subprocess.run([os.path.join(LLVM, "llvm-objdump"), "-d", "--no-show-raw-insn",
+                           "--disassemble-symbols=" + kernel[".name"], kernel["object"]], check=True,
+                          capture_output=True, text=True).stdout
+    return [line.split("//")[0].split() for line in text.split("\n") if line.startswith("\t")]
+
+
+@pytest.mark.parametrize("ring", ["7, 7", "7, 8", "8, 8", "8, 9"])
+def test_wide_conversions_keep_loads_in_flight(kernels, ring):
+    """The 128-bit sums of more than seven inputs: residues are requested in groups of eight, not one by one with a wait
+    for each (an eight-input conversion then waits for memory 16 times an input instead of twice)."""
+    alone = run = 0
+    for op in _instructions(kernels["k_bconv_cols<%s, 2>" % ring]):
+        if op[0] == "global_load_dwordx2":
+            run += 1
+        elif op[0] == "s_waitcnt" and "vmcnt" in " ".join(op):
+            alone += run == 1
+            run = 0
+    assert alone < 8
