@@ -641,6 +641,17 @@ struct RowStage {
     }
 };
 
+// The stage of a rows pass over whole batches: with the integer entries while
+// four workgroups of a tile and its stage fit a CU's 160 KiB of LDS.  They do not
+// at N = 2^13 and 2^14 (32 rows of 128: 43.0 KB), where three then leave the
+// compiler 168 registers and a SIMD 3 waves, in FP64 tiles too (35 limbs x 8
+// polys at N = 2^14, staged / table / with Shoup butterflies, us: forward 50-bit
+// 42.3 / 38.3 / 38.8, 55-bit 52.9 / 49.6 / 49.5; inverse 39.4 / 38.4 / 38.4 and
+// 48.3 / 49.5 / 51.8).
+template <int S1, int S2, int R>
+using PassStage = RowStage<S1, S2, R, (Sub<S2>::LE <= 4 &&
+                                       4 * (8 * R * Geo<S1, S2>::ROW_PITCH + 16 * R * Sub<S2>::E) <= 160 * 1024)>;
+
 // ================================================================ forward
 // Columns pass: src (canonical) -> dst (intermediate form).
 template <int S1, int S2>
@@ -821,7 +832,7 @@ __global__ void __launch_bounds__(R * Sub<S2>::T) __attribute__((amdgpu_waves_pe
 ntt_fwd_rows(NttBatch b, NttTables t) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
-    using RS = RowStage<S1, S2, R>;
+    using RS = PassStage<S1, S2, R>;
     constexpr uint32_t TILES = G::N1 / R;
     __shared__ double lds[R * G::ROW_PITCH];
     __shared__ ulonglong2 twl[RS::N];
@@ -974,7 +985,7 @@ __global__ void __launch_bounds__(R * Sub<S2>::T) __attribute__((amdgpu_waves_pe
 ntt_inv_rows_staged(NttBatch b, NttTables t) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
-    using RS = RowStage<S1, S2, R>;
+    using RS = PassStage<S1, S2, R>;
     constexpr uint32_t TILES = G::N1 / R;
     __shared__ double lds[R * G::ROW_PITCH];
     __shared__ ulonglong2 twl[RS::N];

@@ -74,3 +74,13 @@ def test_wide_conversions_keep_loads_in_flight(kernels, ring):
             alone += run == 1
             run = 0
     assert alone < 8
+
+
+@pytest.mark.parametrize("kernel", ["ntt_fwd_rows<6, 7, 32>", "ntt_fwd_rows<7, 7, 32>", "ntt_fwd_rows<7, 8, 8>",
+                                    "ntt_fwd_rows<8, 8, 8>"])
+def test_forward_rows_occupancy(kernels, kernel):
+    """Four waves on each of a CU's SIMDs (512 registers a lane, 160 KiB of LDS a CU), integer primes or not."""
+    k = kernels[kernel]
+    waves = int(k[".max_flat_workgroup_size"]) // 64
+    assert 16 // waves * int(k[".group_segment_fixed_size"]) <= 160 * 1024
+    assert int(k[".vgpr_count"]) <= 128
