@@ -374,8 +374,8 @@ k_bconv_cols(BconvCols a, NttTables t) {
     __shared__ double lds[G::COL_LDS];
     __shared__ ulonglong2 twl[G::N1];  // the target prime's columns-pass twiddles
     const uint32_t NG = a.batch * a.groups * G::COL_TILES;
-    const uint32_t total = grouped_total(NG, a.J);
-    for (uint32_t p = blockIdx.x; p < total; p += gridDim.x) {
+    const uint32_t total = grouped_total(NG, a.J), step = grid_step();
+    for (uint32_t p = blockIdx.x; p < total; p += step) {
         const uint32_t w = a.sched ? ld_const(a.sched + p) : p;
         uint32_t gt, j;
         if (!grouped_item(w, NG, a.J, gt, j)) continue;
@@ -966,15 +966,15 @@ k_inner_ws(InnerRows a0, NttTables t) {
     __shared__ uint32_t s_last;
     ulonglong2 *tws = reinterpret_cast<ulonglong2 *>(lds + (W::USE_TAB ? W::ROWS * Geo<S1, S2>::ROW_PITCH : W::LDS));
     const uint32_t total = a0.batch * a0.QlP * W::TILES;
-    const uint32_t full = a0.full < total ? a0.full : total;
+    const uint32_t full = a0.full < total ? a0.full : total, step = grid_step();
     constexpr size_t PS = (size_t)2 * W::ROWS * Geo<S1, S2>::N2;
-    const uint32_t g = gridDim.x - 1 - blockIdx.x;
+    const uint32_t g = step - 1 - blockIdx.x;
     const uint32_t u = g / kXcds, c = u % a0.kch;
     const uint32_t j = (u / a0.kch) * kXcds + g % kXcds;
     const uint64_t *parts = a0.partial + (size_t)j * a0.kch * PS;
     // one call for whole items and the chunk: two copies of the item's code
     // did not fit the instruction cache together
-    for (uint32_t i = blockIdx.x;; i += gridDim.x) {
+    for (uint32_t i = blockIdx.x;; i += step) {
         const bool whole = i < full;
         if (!whole && j >= a0.rem) return;
         ws_item<S1, S2>(a0, t, whole ? full - 1 - i : full + j,  // the last items (the longest) first
@@ -1113,8 +1113,8 @@ k_epi_rows(EpiRows a, NttTables t) {
     __shared__ double lds[FG::LDS];
     __shared__ ulonglong2 twl[RowStage<S1, S2, FG::ROWS>::N];
     const uint32_t rr = threadIdx.x / Sub<S2>::T;
-    const uint32_t total = a.M * a.J * FG::TILES;
-    for (uint32_t p = blockIdx.x; p < total; p += gridDim.x) {
+    const uint32_t total = a.M * a.J * FG::TILES, step = grid_step();
+    for (uint32_t p = blockIdx.x; p < total; p += step) {
         const uint32_t w = a.sched ? ld_const(a.sched + p) : p;
         const uint32_t tile = w % FG::TILES, mj = w / FG::TILES;
         const uint32_t m = mj % a.M, j = mj / a.M;

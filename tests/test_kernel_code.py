@@ -84,3 +84,12 @@ def test_forward_rows_occupancy(kernels, kernel):
     waves = int(k[".max_flat_workgroup_size"]) // 64
     assert 16 // waves * int(k[".group_segment_fixed_size"]) <= 160 * 1024
     assert int(k[".vgpr_count"]) <= 128
+
+
+@pytest.mark.parametrize("kernel", ["ntt_fwd_cols<6, 7>", "ntt_fwd_rows<6, 7, 32>", "ntt_inv_rows<6, 7, 32>",
+                                    "ntt_inv_rows_staged<6, 7, 32>", "ntt_inv_cols<6, 7>", "ntt_inv_cols<8, 8>"])
+def test_persistent_loops_keep_the_grid_size(kernels, kernel):
+    """The loop over tiles reads no launch argument between two tiles: its step, the grid's size, is in a register (the
+    one-word scalar loads; the tables a tile reads have entries of two words and more)."""
+    ops = [op[0] for op in _instructions(kernels[kernel])]
+    assert "s_load_dword" not in ops[ops.index("s_barrier"):]
