@@ -95,6 +95,10 @@ struct BconvCols {
     // the inputs of primes of 50 bits or more are stored as 30-bit halves
     // (hi 2^32 + lo), NttLaunch::split30
     uint32_t split30 = 0;
+    // bit g mod 64: group g (or another of that bit) has an input of such a
+    // prime; set by the launcher (kLimbs).  Found from the primes by every item,
+    // with one scalar load after the other, it held up the item's first request.
+    uint64_t wide = 0;
     // position -> item table (a permutation of the launch's positions) built
     // for sched_grid workgroups over sched_total positions; the launcher drops
     // it when its launch differs.  null: position p runs item p
@@ -102,7 +106,7 @@ struct BconvCols {
     uint32_t sched_grid = 0, sched_total = 0;
 };
 
-__device__ __forceinline__ uint32_t bconv_in_row(const BconvCols &a, uint32_t row0, uint32_t i) {
+__host__ __device__ __forceinline__ uint32_t bconv_in_row(const BconvCols &a, uint32_t row0, uint32_t i) {
     if (a.first_row == ~0u) return row0 + i;
     return i == 0 ? a.first_row : row0 + i - 1;
 }
@@ -206,7 +210,8 @@ __device__ __forceinline__ void bconv_limbs(const BconvCols &a, const NttTables 
 // when every input sum stays below 2^64).  One kernel each: in one kernel the
 // branches' values together did not fit the registers, and the few spilled
 // ones, reloaded once an item, waited behind the stores of the item before
-// (L = 35 conversions 242 -> 285 us).
+// (L = 35 conversions 242 -> 285 us).  kOne and kLimbs spill nothing; kWide still
+// spills one staged twiddle (20 bytes).
 enum BconvKind { kOne, kLimbs, kWide };
 
 template <class A, int S1, int S2, int KIND>
@@ -259,10 +264,7 @@ __device__ __forceinline__ void bconv_source(const BconvCols &a, const NttTables
         // an input of a wide prime takes two FP64 products (16 instructions),
         // a narrow one 9; by limbs either takes 4 to 6, and the two Montgomery
         // steps 14 an element: limbs as soon as one input is wide
-        bool limbs = !A::kF64;
-        if constexpr (A::kF64)
-            for (uint32_t i = 0; i < n_in; i++) limbs = limbs || mod_of(i) >= kF64PrimeBound;
-        if (limbs) {
+        if (!A::kF64 || ((a.wide >> (g & 63u)) & 1u)) {
             if constexpr (A::kF64) {
                 bconv_limbs<S1, S2>(a, t, (uint64_t)ar.q, g, j, prow, n_in, row0, in, off, v);
 #pragma unroll
@@ -1290,6 +1292,11 @@ void launch_bconv(const Ctx &c, const BconvCols &a0, hipStream_t s) {
     // every input is below the context's largest prime
     a.mont = c.mont;
     a.sum128 = c.max_modulus <= ~0ull / std::max(a.n_in, a.n_in_last);
+    a.wide = 0;
+    for (uint32_t g = 0; g < (a.in_row_step ? a.groups : 1); ++g)
+        for (uint32_t i = 0; i < (g + 1 == a.groups ? a.n_in_last : a.n_in); ++i)
+            if (c.moduli[bconv_in_row(a, a.in_row0 + g * a.in_row_step, i)] >= kF64PrimeBound)
+                a.wide |= a.in_row_step ? 1ull << (g & 63) : ~0ull;
     const uint32_t total = grouped_total(a.batch * a.groups * G::COL_TILES, a.J);
     const uint32_t grid = fgrid(c, total, 4);
     if (a.sched && (grid != a.sched_grid || total != a.sched_total)) a.sched = nullptr;
@@ -1650,7 +1657,9 @@ void fused_moddown_rescale(const Ctx &c, uint32_t chain, const uint64_t *cx, con
     inv.split = 1;
     inv.split_base = c.Q;
     inv.scale = lv.mdr_scale;
-    inv.split30 = limb_sums(c, alpha + 1);
+    bool wide = c.moduli[Ql - 1] >= kF64PrimeBound;  // else nothing is split, and k_mdr_last has nothing to join
+    for (uint32_t i = 0; i < alpha; ++i) wide = wide || c.moduli[c.Q + i] >= kF64PrimeBound;
+    inv.split30 = wide && limb_sums(c, alpha + 1);
     ntt_inverse(c, inv, s);
     hipLaunchKernelGGL(k_mdr_last, dim3((M * c.N + 255) / 256), dim3(256), 0, s, x, lv.mdr_glast, c.mod, c.ratio,
                        Ql - 1, c.Q, alpha, c.N, M, inv.split30 ? 1u : 0u);

@@ -69,6 +69,8 @@ def _chain(N, kind, nq, alpha):
     """Data primes then special primes of a kind."""
     if kind == "wide":  # all just below 2^60
         return _primes(N, 1 << 60, nq + alpha, True)
+    if kind == "small":  # all just below 2^50
+        return _primes(N, 1 << 50, nq + alpha, True)
     if kind == "mixed":  # narrow and wide data primes in turn, wide special ones
         w, n = _primes(N, 1 << 60, nq + alpha, True), _primes(N, 1 << 50, nq, True)
         return [(w if i % 3 == 0 else n)[i] for i in range(nq)] + w[nq:]
@@ -77,7 +79,7 @@ def _chain(N, kind, nq, alpha):
     return _primes(N, 1 << 61, nq + alpha, True)  # "tight": above 2^60
 
 
-@pytest.mark.parametrize("kind", ["wide", "mixed", "narrow", "tight"])
+@pytest.mark.parametrize("kind", ["wide", "mixed", "narrow", "small", "tight"])
 @pytest.mark.parametrize("nq,alpha", [(3, 1), (4, 2), (12, 6), (14, 7), (8, 8)])
 @pytest.mark.parametrize("logN", [10, 13])
 def test_conversions_edge(dev, logN, nq, alpha, kind):

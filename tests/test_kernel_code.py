@@ -93,3 +93,13 @@ def test_persistent_loops_keep_the_grid_size(kernels, kernel):
     one-word scalar loads; the tables a tile reads have entries of two words and more)."""
     ops = [op[0] for op in _instructions(kernels[kernel])]
     assert "s_load_dword" not in ops[ops.index("s_barrier"):]
+
+
+@pytest.mark.parametrize("ring", ["6, 7", "7, 7", "7, 8", "8, 8", "8, 9"])
+@pytest.mark.parametrize("kind", [0, 1])
+def test_conversions_in_registers(kernels, ring, kind):
+    """Single inputs and sums of 30-bit limbs fit the registers of four waves a SIMD with nothing spilled: a spilled
+    value, reloaded once an item, waits behind the stores of the item before."""
+    k = kernels["k_bconv_cols<%s, %d>" % (ring, kind)]
+    assert int(k[".private_segment_fixed_size"]) == 0
+    assert int(k[".vgpr_count"]) <= 128
