@@ -55,18 +55,34 @@ constexpr int half_rows() {
     return S2 == 8 && G::ROWS == 16 ? 8 : G::ROWS;
 }
 
+// Whether a launch whose integer stage costs a workgroup a CU (kIntStageCosts)
+// takes the kernel with it: never without integer primes; with them, if its tiles
+// are at most `all`.  Forward, all: the tiles that three workgroups a CU hold at
+// once; a fourth has work only beyond them, and up to there the table's latency
+// counts (with the stage / without, us: N = 2^13, 4 limbs of 60-bit primes 13.0 /
+// 13.7, 50 limbs 14.5 / 15.2, 560 limbs 53.8 / 50.8; 50-bit primes 10.1 / 9.9,
+// 12.6 / 12.4, 42.4 / 39.3; 2^14, 280 limbs 53.8 / 49.9).  The inverse pass runs 3
+// waves a SIMD in either form, so integer primes always take it (2^14, 280 limbs
+// 48.2 / 49.4; 50-bit primes 39.4 / 37.8).
+bool pass_staged(const Ctx &c, const NttBatch &b, uint32_t tiles, uint32_t all) {
+    for (uint32_t l = 0; l < b.L; ++l)
+        if (c.moduli[b.map.row(l)] >= kF64PrimeBound) return tiles <= all;
+    return false;
+}
+
 // the forward rows pass alone: b.src holds a columns pass's output
 template <int S1, int S2>
 void fwd_rows(const Ctx &c, const NttBatch &b, const NttTables &t, hipStream_t s) {
     using G = Geo<S1, S2>;
-    const uint32_t ml = b.M * b.L;
-    constexpr int RH = half_rows<S1, S2>();
-    if (RH != G::ROWS)
-        hipLaunchKernelGGL((ntt_fwd_rows<S1, S2, RH>), dim3(grid_for(c, ml * (G::N1 / RH), c.ntt_wpc_fwd * (G::ROWS / RH))),
-                           dim3(RH * Sub<S2>::T), 0, s, b, t);
-    else
-        hipLaunchKernelGGL((ntt_fwd_rows<S1, S2>), dim3(grid_for(c, ml * G::ROW_TILES, c.ntt_wpc_fwd)), dim3(G::ROW_THREADS), 0, s, b,
-                           t);
+    constexpr int R = half_rows<S1, S2>();
+    const uint32_t tiles = b.M * b.L * (G::N1 / R);
+    const dim3 grid(grid_for(c, tiles, c.ntt_wpc_fwd * (G::ROWS / R))), block(R * Sub<S2>::T);
+    if constexpr (kIntStageCosts<S1, S2, R>)
+        if (!pass_staged(c, b, tiles, (uint32_t)c.n_cu * 3)) {
+            hipLaunchKernelGGL((ntt_fwd_rows<S1, S2, R, false>), grid, block, 0, s, b, t);
+            return;
+        }
+    hipLaunchKernelGGL((ntt_fwd_rows<S1, S2, R>), grid, block, 0, s, b, t);
 }
 
 template <int S1, int S2>
@@ -96,10 +112,13 @@ template <int S1, int S2>
 void inv(const Ctx &c, const NttBatch &b, const NttTables &t, hipStream_t s) {
     using G = Geo<S1, S2>;
     const uint32_t ml = b.M * b.L;
-    if (ml >= kInvStagedLimbs)
-        hipLaunchKernelGGL((ntt_inv_rows_staged<S1, S2>), dim3(grid_for(c, ml * G::ROW_TILES, 3)),
-                           dim3(G::ROW_THREADS), 0, s, b, t);
-    else if (half_rows<S1, S2>() != G::ROWS)
+    if (ml >= kInvStagedLimbs) {
+        const dim3 grid(grid_for(c, ml * G::ROW_TILES, 3)), block(G::ROW_THREADS);
+        if (kIntStageCosts<S1, S2, G::ROWS> && !pass_staged(c, b, 0, 0))
+            hipLaunchKernelGGL((ntt_inv_rows_staged<S1, S2, G::ROWS, false>), grid, block, 0, s, b, t);
+        else
+            hipLaunchKernelGGL((ntt_inv_rows_staged<S1, S2>), grid, block, 0, s, b, t);
+    } else if (half_rows<S1, S2>() != G::ROWS)
         hipLaunchKernelGGL((ntt_inv_rows<S1, S2, half_rows<S1, S2>()>),
                            dim3(grid_for(c, ml * (G::N1 / half_rows<S1, S2>()), c.ntt_wpc * (G::ROWS / half_rows<S1, S2>()))),
                            dim3(half_rows<S1, S2>() * Sub<S2>::T), 0, s, b, t);

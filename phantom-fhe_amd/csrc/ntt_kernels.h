@@ -33,7 +33,7 @@ namespace pfa {
 // Which physical table row (prime) a batch limb uses; see NttBatch.
 struct LimbMap {
     uint32_t start, split, split_base;
-    __device__ __forceinline__ uint32_t row(uint32_t l) const {
+    __host__ __device__ __forceinline__ uint32_t row(uint32_t l) const {
         return l < split ? start + l : split_base + (l - split);
     }
 };
@@ -653,16 +653,14 @@ struct RowStage {
     }
 };
 
-// The stage of a rows pass over whole batches: with the integer entries while
-// four workgroups of a tile and its stage fit a CU's 160 KiB of LDS.  They do not
-// at N = 2^13 and 2^14 (32 rows of 128: 43.0 KB), where three then leave the
-// compiler 168 registers and a SIMD 3 waves, in FP64 tiles too (35 limbs x 8
-// polys at N = 2^14, staged / table / with Shoup butterflies, us: forward 50-bit
-// 42.3 / 38.3 / 38.8, 55-bit 52.9 / 49.6 / 49.5; inverse 39.4 / 38.4 / 38.4 and
-// 48.3 / 49.5 / 51.8).
+// Rows passes over whole batches have a variant that stages no integer entries
+// (INT false) where four workgroups of a tile and its integer stage do not fit a
+// CU's 160 KiB of LDS: N = 2^13 and 2^14, 32 rows of 128, 43.0 KB instead of 39.4.
+// Three workgroups a CU then leave the compiler 168 registers and a SIMD 3 waves,
+// in FP64 tiles too; the launcher chooses (pass_staged).
 template <int S1, int S2, int R>
-using PassStage = RowStage<S1, S2, R, (Sub<S2>::LE <= 4 &&
-                                       4 * (8 * R * Geo<S1, S2>::ROW_PITCH + 16 * R * Sub<S2>::E) <= 160 * 1024)>;
+constexpr bool kIntStageCosts =
+    Sub<S2>::LE <= 4 && 4 * (8 * R * Geo<S1, S2>::ROW_PITCH + 16 * R * Sub<S2>::E) > 160 * 1024;
 
 // ================================================================ forward
 // Columns pass: src (canonical) -> dst (intermediate form).
@@ -839,12 +837,12 @@ __device__ __forceinline__ const uint64_t *rows_ptr(const NttBatch &b, const Til
     return base + r.m * stride + (size_t)r.l * G::N + (size_t)(r.tile * R + rr) * G::N2;
 }
 
-template <int S1, int S2, int R = Geo<S1, S2>::ROWS>
+template <int S1, int S2, int R = Geo<S1, S2>::ROWS, bool INT = (Sub<S2>::LE <= 4)>
 __global__ void __launch_bounds__(R * Sub<S2>::T) __attribute__((amdgpu_waves_per_eu(4, 8)))
 ntt_fwd_rows(NttBatch b, NttTables t) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
-    using RS = PassStage<S1, S2, R>;
+    using RS = RowStage<S1, S2, R, INT>;
     constexpr uint32_t TILES = G::N1 / R;
     __shared__ double lds[R * G::ROW_PITCH];
     __shared__ ulonglong2 twl[RS::N];
@@ -992,12 +990,12 @@ __global__ void __launch_bounds__(R * Sub<S2>::T) ntt_inv_rows(NttBatch b, NttTa
 // Faster on large batches (config-2 inverse 44.5-44.9 -> 41.3 us), slightly
 // slower on the few-limb transforms of a key switch, so ntt_inverse picks it
 // by batch size.
-template <int S1, int S2, int R = Geo<S1, S2>::ROWS>
+template <int S1, int S2, int R = Geo<S1, S2>::ROWS, bool INT = (Sub<S2>::LE <= 4)>
 __global__ void __launch_bounds__(R * Sub<S2>::T) __attribute__((amdgpu_waves_per_eu(3, 8)))
 ntt_inv_rows_staged(NttBatch b, NttTables t) {
     using G = Geo<S1, S2>;
     using SB = Sub<S2>;
-    using RS = PassStage<S1, S2, R>;
+    using RS = RowStage<S1, S2, R, INT>;
     constexpr uint32_t TILES = G::N1 / R;
     __shared__ double lds[R * G::ROW_PITCH];
     __shared__ ulonglong2 twl[RS::N];

@@ -65,6 +65,31 @@ def test_ntt_edge_primes(dev, logN):
         assert all(np.array_equal(g, want) for g in got), first_mismatch(got[0], want)
 
 
+@pytest.mark.parametrize("logN", [13, 14])
+@pytest.mark.parametrize("kind", ["narrow", "wide", "mixed"])
+def test_rows_passes_with_and_without_stage(dev, logN, kind):
+    """N = 2^13 and 2^14: the forward rows pass with integer twiddles in LDS up to three tiles a CU, without beyond and
+    for 50-bit primes alone; the inverse one with them for any integer prime from 48 limbs on."""
+    import pfa_native as P
+    import torch
+
+    N = 1 << logN
+    narrow, wide = _primes(N, 1 << 50, 3, True), _primes(N, 1 << 60, 3, True)
+    mods = {"narrow": narrow, "wide": wide, "mixed": narrow[:2] + wide[:1]}[kind]
+    ctx, orc = P.NativeContext(N, mods, 1), O.Oracle(N, mods, 1)
+    x = _extremes(np.random.default_rng(logN), mods, N)
+    tiles = N // 128 // 32  # of a limb: rows of 128, 32 a tile
+    most = torch.cuda.get_device_properties(dev).multi_processor_count * 3 // tiles // len(mods)  # polys
+    for batch in (4, 16, most, most + 1):
+        y = np.concatenate([x] * (batch // 4 + 1))[:batch]
+        for transform, check in ((ctx.ntt_forward, orc.ntt_fwd), (ctx.ntt_inverse, orc.ntt_inv)):
+            d = to_dev(y, dev)
+            transform(d, batch, len(mods), 0)
+            want, got = check(x), to_host(d)
+            for k in range(batch):
+                assert np.array_equal(got[k], want[k % 4]), (batch, k, first_mismatch(got[k], want[k % 4]))
+
+
 def _chain(N, kind, nq, alpha):
     """Data primes then special primes of a kind."""
     if kind == "wide":  # all just below 2^60
@@ -79,9 +104,14 @@ def _chain(N, kind, nq, alpha):
     return _primes(N, 1 << 61, nq + alpha, True)  # "tight": above 2^60
 
 
-@pytest.mark.parametrize("kind", ["wide", "mixed", "narrow", "small", "tight"])
-@pytest.mark.parametrize("nq,alpha", [(3, 1), (4, 2), (12, 6), (14, 7), (8, 8)])
-@pytest.mark.parametrize("logN", [10, 13])
+_SHAPES = [(logN, nq, alpha, kind) for logN in (10, 13) for nq, alpha in ((3, 1), (4, 2), (12, 6), (14, 7), (8, 8))
+           for kind in ("wide", "mixed", "narrow", "small", "tight")]
+# rounds of 16 and 32 elements, and the inner product without staged twiddles (N = 2^17)
+_SHAPES += [(logN, nq, alpha, kind) for logN in (14, 16, 17) for nq, alpha in ((4, 2), (8, 8))
+            for kind in ("mixed", "tight")]
+
+
+@pytest.mark.parametrize("logN,nq,alpha,kind", _SHAPES)
 def test_conversions_edge(dev, logN, nq, alpha, kind):
     """multiply, relinearize and rescale (the fused conversion of alpha + 1
     inputs), then relinearize alone (ModUp and ModDown of alpha inputs), at the

@@ -47,8 +47,8 @@ def kernels(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize("kernel", ["ntt_fwd_rows<8, 9, 8>", "ntt_inv_rows<8, 9, 8>", "ntt_inv_rows_staged<8, 9, 8>",
-                                    "ntt_fwd_cols<8, 9>", "ntt_inv_cols<8, 9>", "k_epi_rows<8, 9>",
+@pytest.mark.parametrize("kernel", ["ntt_fwd_rows<8, 9, 8, false>", "ntt_inv_rows<8, 9, 8>",
+                                    "ntt_inv_rows_staged<8, 9, 8, false>", "ntt_fwd_cols<8, 9>", "ntt_inv_cols<8, 9>", "k_epi_rows<8, 9>",
                                     "k_inner_ws<8, 9>"])
 def test_largest_ring_elements_in_registers(kernels, kernel):
     """N = 2^17: 32 elements a thread (64 sums in the inner product), the longest unrolled loops."""
@@ -76,18 +76,21 @@ def test_wide_conversions_keep_loads_in_flight(kernels, ring):
     assert alone < 8
 
 
-@pytest.mark.parametrize("kernel", ["ntt_fwd_rows<6, 7, 32>", "ntt_fwd_rows<7, 7, 32>", "ntt_fwd_rows<7, 8, 8>",
-                                    "ntt_fwd_rows<8, 8, 8>"])
+@pytest.mark.parametrize("kernel", ["ntt_fwd_rows<6, 7, 32, false>", "ntt_fwd_rows<7, 7, 32, false>",
+                                    "ntt_fwd_rows<7, 8, 8, true>", "ntt_fwd_rows<8, 8, 8, true>"])
 def test_forward_rows_occupancy(kernels, kernel):
-    """Four waves on each of a CU's SIMDs (512 registers a lane, 160 KiB of LDS a CU), integer primes or not."""
+    """The forward rows pass of large batches: four waves on each of a CU's SIMDs (512 registers a lane, 160 KiB of LDS a
+    CU), integer primes or not."""
     k = kernels[kernel]
     waves = int(k[".max_flat_workgroup_size"]) // 64
     assert 16 // waves * int(k[".group_segment_fixed_size"]) <= 160 * 1024
     assert int(k[".vgpr_count"]) <= 128
 
 
-@pytest.mark.parametrize("kernel", ["ntt_fwd_cols<6, 7>", "ntt_fwd_rows<6, 7, 32>", "ntt_inv_rows<6, 7, 32>",
-                                    "ntt_inv_rows_staged<6, 7, 32>", "ntt_inv_cols<6, 7>", "ntt_inv_cols<8, 8>"])
+@pytest.mark.parametrize("kernel", ["ntt_fwd_cols<6, 7>", "ntt_fwd_rows<6, 7, 32, false>",
+                                    "ntt_fwd_rows<6, 7, 32, true>", "ntt_inv_rows<6, 7, 32>",
+                                    "ntt_inv_rows_staged<6, 7, 32, true>", "ntt_inv_cols<6, 7>",
+                                    "ntt_inv_cols<8, 8>"])
 def test_persistent_loops_keep_the_grid_size(kernels, kernel):
     """The loop over tiles reads no launch argument between two tiles: its step, the grid's size, is in a register (the
     one-word scalar loads; the tables a tile reads have entries of two words and more)."""
