@@ -95,10 +95,10 @@ struct BconvCols {
     // the inputs of primes of 50 bits or more are stored as 30-bit halves
     // (hi 2^32 + lo), NttLaunch::split30
     uint32_t split30 = 0;
-    // bit g mod 64: group g (or another of that bit) has an input of such a
-    // prime; set by the launcher (kLimbs).  Found from the primes by every item,
-    // with one scalar load after the other, it held up the item's first request.
-    uint64_t wide = 0;
+    // some group has an input of such a prime (set by the launcher): else kLimbs
+    // items need not look at their inputs' primes, one scalar load after the
+    // other before the first request
+    uint32_t wide = 0;
     // position -> item table (a permutation of the launch's positions) built
     // for sched_grid workgroups over sched_total positions; the launcher drops
     // it when its launch differs.  null: position p runs item p
@@ -264,7 +264,11 @@ __device__ __forceinline__ void bconv_source(const BconvCols &a, const NttTables
         // an input of a wide prime takes two FP64 products (16 instructions),
         // a narrow one 9; by limbs either takes 4 to 6, and the two Montgomery
         // steps 14 an element: limbs as soon as one input is wide
-        if (!A::kF64 || ((a.wide >> (g & 63u)) & 1u)) {
+        bool limbs = !A::kF64;
+        if constexpr (A::kF64)
+            if (a.wide)
+                for (uint32_t i = 0; i < n_in; i++) limbs = limbs || mod_of(i) >= kF64PrimeBound;
+        if (limbs) {
             if constexpr (A::kF64) {
                 bconv_limbs<S1, S2>(a, t, (uint64_t)ar.q, g, j, prow, n_in, row0, in, off, v);
 #pragma unroll
@@ -1295,8 +1299,7 @@ void launch_bconv(const Ctx &c, const BconvCols &a0, hipStream_t s) {
     a.wide = 0;
     for (uint32_t g = 0; g < (a.in_row_step ? a.groups : 1); ++g)
         for (uint32_t i = 0; i < (g + 1 == a.groups ? a.n_in_last : a.n_in); ++i)
-            if (c.moduli[bconv_in_row(a, a.in_row0 + g * a.in_row_step, i)] >= kF64PrimeBound)
-                a.wide |= a.in_row_step ? 1ull << (g & 63) : ~0ull;
+            if (c.moduli[bconv_in_row(a, a.in_row0 + g * a.in_row_step, i)] >= kF64PrimeBound) a.wide = 1;
     const uint32_t total = grouped_total(a.batch * a.groups * G::COL_TILES, a.J);
     const uint32_t grid = fgrid(c, total, 4);
     if (a.sched && (grid != a.sched_grid || total != a.sched_total)) a.sched = nullptr;

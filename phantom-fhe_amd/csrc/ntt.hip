@@ -114,10 +114,14 @@ void inv(const Ctx &c, const NttBatch &b, const NttTables &t, hipStream_t s) {
     const uint32_t ml = b.M * b.L;
     if (ml >= kInvStagedLimbs) {
         const dim3 grid(grid_for(c, ml * G::ROW_TILES, 3)), block(G::ROW_THREADS);
-        if (kIntStageCosts<S1, S2, G::ROWS> && !pass_staged(c, b, 0, 0))
-            hipLaunchKernelGGL((ntt_inv_rows_staged<S1, S2, G::ROWS, false>), grid, block, 0, s, b, t);
-        else
+        if constexpr (kIntStageCosts<S1, S2, G::ROWS>) {
+            if (pass_staged(c, b, 0, 0))
+                hipLaunchKernelGGL((ntt_inv_rows_staged<S1, S2>), grid, block, 0, s, b, t);
+            else
+                hipLaunchKernelGGL((ntt_inv_rows_staged<S1, S2, G::ROWS, false>), grid, block, 0, s, b, t);
+        } else {
             hipLaunchKernelGGL((ntt_inv_rows_staged<S1, S2>), grid, block, 0, s, b, t);
+        }
     } else if (half_rows<S1, S2>() != G::ROWS)
         hipLaunchKernelGGL((ntt_inv_rows<S1, S2, half_rows<S1, S2>()>),
                            dim3(grid_for(c, ml * (G::N1 / half_rows<S1, S2>()), c.ntt_wpc * (G::ROWS / half_rows<S1, S2>()))),
