@@ -415,8 +415,11 @@ static Sched cached_schedule(const Ctx &c, const std::array<uint32_t, 4> &key, u
     return sc;
 }
 
-// An integer-policy target (a prime of 50 bits or more: Montgomery sums and
-// Shoup butterflies) costs about three FP64 ones.
+// An integer-policy target (a prime of 50 bits or more) weighs three FP64 ones: a
+// butterfly takes 73 cycles against 42, and the other work of an item (conversion,
+// epilogue) more than that.  The lists are not sensitive to it: weights of 2 and 3
+// measure the same to 0.5% (20 + 4, 24 + 4 and 12 + 3 primes, N = 2^13 to 2^17); with
+// equal ones rotations over 20 + 4 primes lose 1.5-2%.
 static uint8_t target_cost(const Ctx &c, uint32_t row) { return c.moduli[row] < kF64PrimeBound ? 1 : 3; }
 
 Sched modup_schedule(const Ctx &c, uint32_t chain, uint32_t batch) {

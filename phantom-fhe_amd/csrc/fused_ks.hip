@@ -35,9 +35,10 @@
 // split t = h 2^32 + l and converted as h [m 2^32]_q + l m.  Each product is
 // within (-0.875 q, 0.875 q) (|t w / q| < 2^50, so fl(t wq) is within 3/8 of
 // the true quotient); the sum is reduced whenever the next product could take
-// it past 7 x 0.875 q, which keeps every partial sum below 2^53.  Targets
-// q >= 2^50, and FP64 targets with a wide input, sum 30-bit limb products
-// (bconv_limbs).
+// it past 7 x 0.875 q, which keeps every partial sum below 2^53.  In conversions
+// of two to seven inputs of primes below 2^60, targets q >= 2^50 and FP64 targets
+// with a wide input sum 30-bit limb products instead (bconv_limbs); beyond,
+// targets q >= 2^50 take 128-bit sums or reduced products (BconvKind).
 #include <algorithm>
 
 #include "internal.h"
@@ -136,14 +137,22 @@ __device__ __forceinline__ const uint64_t *bconv_next(const uint64_t *in, uint32
 }
 
 constexpr uint32_t kLimbInputs = 7;
+// the middle sum of n inputs, limbs of 2^30 - 1, in bconv_limbs
+constexpr bool limb_sum_fits(uint32_t n) {
+    constexpr unsigned __int128 L = (1u << 30) - 1;
+    return (2 * n + 2) * L * L + ((n + 1) * L * L >> 30) < (unsigned __int128)1 << 64;
+}
+static_assert(limb_sum_fits(kLimbInputs) && !limb_sum_fits(kLimbInputs + 1));
 
 // sum_i t_i m_i mod q, in [0, (n_in + 1) q), for elements F + T e of the
 // thread's column, by 30-bit limbs: t = t1 2^30 + t0 and the factor in
 // Montgomery form, m 2^60 mod q = m1 2^30 + m0, so a product is four 32-bit
 // multiply-adds into three 64-bit sums, with no carries to move (a 128-bit sum
 // takes about 13 instructions a product); two 30-bit Montgomery steps then
-// divide by 2^60.  With t, q < 2^60 and n <= 7: the middle sum stays below
-// (2 n + 1) 2^60 + 2^35 < 2^64 and the result below n q^2 / 2^60 + q.
+// divide by 2^60.  Every limb is at most 2^30 - 1 (t, q < 2^60).  The middle sum
+// takes 2 n products, two more of the steps and a carry below 2^33:
+// (2 n + 2) (2^30 - 1)^2 + 2^33 < 2^64 for n <= 7 and no more (kLimbInputs).  The
+// result is below n q^2 / 2^60 + q.
 // Inputs of wide primes come split from the INTT; narrower ones are split here.
 // Measured at N = 2^16 with the columns pass it feeds: 14 polys of 6 wide inputs to
 // 28 wide targets plus 5 digits of 6 to 34, 322 us with 128-bit sums, 270 us.

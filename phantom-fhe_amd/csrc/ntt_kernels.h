@@ -568,19 +568,18 @@ struct TileTw {
     static constexpr bool kStaged = false;
 };
 
-// The same with the factors in LDS: rb and small point there, and ra at the
-// row's first-round entries (LdsTwA, integer policy).
+// The same with the first-round integer entries in LDS, too: ra points at the
+// row's (LdsTwA).
 struct StagedTw : TileTw {
     const ulonglong2 *ra;
     static constexpr bool kStaged = true;
 };
 
 template <int S1, int S2>
-__device__ __forceinline__ TileTw global_tw(const NttTables &t, uint32_t prow, uint32_t k1, bool fwd) {
+__device__ __forceinline__ TileTw global_inv_tw(const NttTables &t, uint32_t prow, uint32_t k1) {
     using G = Geo<S1, S2>;
-    const ulonglong2 *tab = (fwd ? t.tw : t.itw) + (size_t)prow * G::N;
-    return TileTw{tab, tab, (fwd ? t.rb_fw : t.rb_inv) + (size_t)prow * S2 * G::N1,
-                  (fwd ? t.small_fw : t.small_inv) + (size_t)prow * kSmall, k1};
+    const ulonglong2 *tab = t.itw + (size_t)prow * G::N;
+    return TileTw{tab, tab, t.rb_inv + (size_t)prow * S2 * G::N1, t.small_inv + (size_t)prow * kSmall, k1};
 }
 
 // A gather of N twiddle entries into LDS, split in two so the caller can issue
@@ -726,7 +725,7 @@ __device__ __forceinline__ void fwd_cols_tile(const uint64_t (&raw)[Sub<S1>::E],
 }
 
 // The forward passes keep no register prefetch: without it they fit 4 waves
-// per SIMD (102 / 126 VGPRs, against 135 / 158 with a prefetched tile at 3),
+// per SIMD (114 / 128 VGPRs; a prefetched tile takes 32 more and leaves 3),
 // and the extra resident workgroups hide the load latency better (measured on
 // the 2 x 35-limb config-2 batch: 43-44.5 -> 40.8-41 us per forward NTT).
 template <int S1, int S2>
@@ -802,13 +801,6 @@ __device__ __forceinline__ void fwd_rows_core(typename A::T (&x)[Sub<S2>::E], co
     __syncthreads();
 #pragma unroll
     for (int e = 0; e < SB::E; e++) x[e] = lr[rpad(F + SB::T * e)];
-}
-
-// the same with the twiddles read from the global tables
-template <class A, int S1, int S2>
-__device__ __forceinline__ void fwd_rows_core(typename A::T (&x)[Sub<S2>::E], const A &ar, const NttTables &t,
-                                              uint32_t prow, uint32_t k1, typename A::T *lr) {
-    fwd_rows_core<A, S1, S2, Geo<S1, S2>::N1>(x, ar, global_tw<S1, S2>(t, prow, k1, true), k1, lr);
 }
 
 template <class A, int S1, int S2, int RBS, int R = Geo<S1, S2>::ROWS, class TW>
@@ -971,7 +963,7 @@ __global__ void __launch_bounds__(R * Sub<S2>::T) ntt_inv_rows(NttBatch b, NttTa
         }
         const uint32_t prow = b.map.row(r.l);
         const uint64_t q = t.mod[prow];
-        const TileTw w = global_tw<S1, S2>(t, prow, r.tile * R + rr, false);
+        const TileTw w = global_inv_tw<S1, S2>(t, prow, r.tile * R + rr);
         uint64_t *olimb = b.dst + r.m * b.dstride + (size_t)r.l * G::N;
         if (q < kF64PrimeBound)
             inv_rows_tile<ArithF64, S1, S2, G::N1, true, R>(raw, w, r, q, lds, olimb);
@@ -986,7 +978,7 @@ __global__ void __launch_bounds__(R * Sub<S2>::T) ntt_inv_rows(NttBatch b, NttTa
 
 // The same pass without register prefetch, its tile's twiddle factors staged
 // in LDS (requested before the residues, so one wait covers both) instead of
-// read from the global tables inside the rounds: 142 VGPRs, 3 waves per SIMD.
+// read from the global tables inside the rounds: 166 VGPRs, 3 waves per SIMD.
 // Faster on large batches (config-2 inverse 44.5-44.9 -> 41.3 us), slightly
 // slower on the few-limb transforms of a key switch, so ntt_inverse picks it
 // by batch size.
@@ -1063,7 +1055,7 @@ __device__ __forceinline__ void inv_cols_tile(const uint64_t (&raw)[Sub<S1>::E],
     }
 }
 
-// Like the forward columns pass: no register prefetch (124 VGPRs, 4 waves
+// Like the forward columns pass: no register prefetch (122 VGPRs, 4 waves
 // per SIMD) and the tile's twiddle factors staged in LDS, requested before its
 // residues (config-2 inverse 41.0-41.2 -> 39.4 us; with the prefetch at 3
 // waves, the staging alone had cost 3 us).
